@@ -77,6 +77,29 @@ def test_gram_hermitian(dtype, m, k):
     assert torch.equal(h, h.conj().T)
 
 
+@pytest.mark.parametrize('dtype', DTYPES)
+@pytest.mark.parametrize('m,n,k', [(1, 1, 8), (64, 64, 20), (64, 33, 1732),
+                                   (5, 64, 4096), (65, 64, 4096),
+                                   (17, 17, 131076)])
+def test_gram_small_band_counts(dtype, m, n, k):
+    """The 64 x 64 form and its edges: one band, ragged rows, a k that ends
+    inside a 128-byte segment, more slices than one block, one row beyond
+    it.  A wave sums at most k / 4 products before the FP64 sums, so the
+    bounds of the other tests hold."""
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m + 3 * n + k)
+    a = torch.randn((m, k), dtype=dtype, device='cuda', generator=g)
+    b = torch.randn((n, k), dtype=dtype, device='cuda', generator=g)
+    c = blas.gram(a, b, alpha=-1.5, conj=True)
+    ref = exact(a, b, -1.5, True)
+    err = (c - ref).abs() / (1.5 * bound(a, b))
+    assert float(err.max()) < tol(dtype)
+    s = blas.gram(a, hermitian=True)
+    ref = exact(a, a, 1.0, False)
+    assert float(((s - ref).abs() / bound(a, a)).max()) < tol(dtype)
+    assert torch.equal(s, s.conj().T)
+
+
 def test_gram_views_and_errors():
     """Row pitch from a strided band view; the C ABI refuses rows that are
     not 16-byte aligned (the Python layer then takes an FP64 GEMM on the
