@@ -52,6 +52,8 @@ _SIGNATURES = {
     'gh_lfc_destroy': (_c.c_int, [P]),
     'gh_lfc_nfunctions': (_c.c_int, [P]),
     'gh_lfc_integrate': (_c.c_int, [P, P, P, I64, _c.c_int, P]),
+    'gh_lfc_integrate_work': (I64, [P, I64]),
+    'gh_lfc_integrate_ws': (_c.c_int, [P, P, P, I64, _c.c_int, P, I64, P]),
     'gh_lfc_add': (_c.c_int, [P, P, P, I64, _c.c_int, P]),
     'gh_lfc_apply_dH': (_c.c_int, [P, P, P, P, P, P, I64, P]),
     'gh_stream_copy': (_c.c_int, [P, P, I64, _c.c_int, P]),

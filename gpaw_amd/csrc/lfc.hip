@@ -71,9 +71,14 @@ template <> struct IntBT<cplx<float>> { static constexpr int value = 8; };
 // function) accumulates sum_e A[e, m] a[x, e] for all bands of the tile,
 // reading whole A rows with coalesced loads.  Group partial sums are
 // reduced through LDS in a fixed order (deterministic).
+// With few atoms x band tiles an atom's chunks are dealt to gridDim.z
+// slices, whose FP64 sums go to `part` (slice, band, M) and are added in
+// slice order by lfc_slices_kernel: a sphere of 4189 points is 17 chunks in
+// a chain of dependent loads of about 3.5 us each.
 template <typename V, typename S>
 __global__ void __launch_bounds__(256)
 lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
+                     typename Wide<V>::type* __restrict__ part,
                      const int64_t* __restrict__ entry_ptr,
                      const int32_t* __restrict__ M_ptr,
                      const int64_t* __restrict__ A_off,
@@ -92,9 +97,16 @@ lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
     const int M0 = M_ptr[atom];
     const int nm = M_ptr[atom + 1] - M0;
     if (nm == 0) return;
-    const int64_t e0 = entry_ptr[atom];
-    const int64_t e1 = entry_ptr[atom + 1];
+    int64_t e0 = entry_ptr[atom];
+    int64_t e1 = entry_ptr[atom + 1];
     const S* __restrict__ Aa = A + A_off[atom];
+    {
+        const int64_t nch = (e1 - e0 + kIntChunk - 1) / kIntChunk, ns = gridDim.z;
+        const int64_t c0 = nch * blockIdx.z / ns, c1 = nch * (blockIdx.z + 1) / ns;
+        Aa += c0 * kIntChunk * nm;
+        e1 = min(e1, e0 + c1 * kIntChunk);
+        e0 += c0 * kIntChunk;
+    }
     const int t = threadIdx.x;
     const int nb = min(BT, nbands - x0);
     const int ngrp = kIntChunk / nm;
@@ -155,8 +167,23 @@ lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
         const int mm = u - b * nm;
         W sum = vzero<W>();
         for (int g = 0; g < ngrp; g++) sum = vadd(sum, Rb[(g * BT + b) * nm + mm]);
-        if (b < nb) narrow(vscale(sum, (double)dv), c + (size_t)(x0 + b) * Mmax + M0 + mm);
+        if (b >= nb) continue;
+        if (part) part[((size_t)blockIdx.z * nbands + x0 + b) * Mmax + M0 + mm] = sum;
+        else narrow(vscale(sum, (double)dv), c + (size_t)(x0 + b) * Mmax + M0 + mm);
     }
+}
+
+// c = dv * sum over the slices (in order) of their sums
+template <typename V>
+__global__ void __launch_bounds__(256)
+lfc_slices_kernel(const typename Wide<V>::type* __restrict__ part, V* __restrict__ c,
+                  int64_t total, int ns, double dv) {
+    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (i >= total) return;
+    typename Wide<V>::type sum = part[i];
+#pragma unroll 4
+    for (int s = 1; s < ns; s++) sum = vadd(sum, part[s * total + i]);
+    narrow(vscale(sum, dv), c + i);
 }
 
 // add: one wavefront per (unit of the colour, chunk of 64 entries, band
@@ -398,6 +425,7 @@ struct gh_lfc {
     int max_nm = 0;                     // most functions on one atom
     int uniform_nm = -1;                // functions per atom if all equal
     int64_t max_unit = 0;               // most entries in one add unit
+    int64_t max_entries = 0;            // most entries of one atom
     int32_t* unit_atom = nullptr;       // add unit -> atom
     int64_t* unit_beg = nullptr;        // add unit -> entry range
     int64_t* unit_end = nullptr;
@@ -565,6 +593,7 @@ int gh_lfc_create(gh_lfc** out, int64_t ngpts, int natoms,
         if (a == 0) h->uniform_nm = nma;
         else if (h->uniform_nm != nma) h->uniform_nm = -1;
         h->max_nm = std::max(h->max_nm, M_ptr[a + 1] - M_ptr[a]);
+        h->max_entries = std::max(h->max_entries, entry_ptr[a + 1] - entry_ptr[a]);
     }
     for (int u = 0; u < nunits; u++)
         h->max_unit = std::max(h->max_unit, unit_end[u] - unit_beg[u]);
@@ -684,8 +713,35 @@ static const void* phase_table(const gh_lfc* h, int q) {
     return (const char*)h->phase_w + (size_t)q * h->nw * 2 * s;
 }
 
+// Slices of each atom's entries.  One slice per atom is enough when atoms x
+// band tiles already give every CU four blocks (what the LDS lets run
+// together); below that the chunks of a sphere are spread until they do.
+// FP64, 24 atoms x 3 tiles of 48 bands: 124 us in one slice, 31 us in 14 and
+// 5 us for their sum; 4 atoms x 4 bands: 59 -> 9 + 4 us.
+static int integrate_slices(const gh_lfc* h, int64_t nbands) {
+    const int64_t bt = h->dtype == GH_C128 ? IntBT<cplx<double>>::value
+                       : h->dtype == GH_C64 ? IntBT<cplx<float>>::value
+                                            : IntBT<double>::value;
+    const int64_t blocks = h->natoms * ((nbands + bt - 1) / bt);
+    const int64_t chunks = (h->max_entries + kIntChunk - 1) / kIntChunk;
+    if (blocks <= 0 || blocks >= 1024) return 1;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(chunks, 1024 / blocks));
+}
+
+int64_t gh_lfc_integrate_work(const gh_lfc* h, int64_t nbands) {
+    if (!h || nbands <= 0) return 0;
+    const int ns = integrate_slices(h, nbands);
+    return ns > 1 ? (int64_t)ns * nbands * h->Mmax * (cplxd(h->dtype) ? 16 : 8) : 0;
+}
+
 int gh_lfc_integrate(const gh_lfc* h, const void* a_dev, void* c_dev,
                      int64_t nbands, int q, void* stream) {
+    return gh_lfc_integrate_ws(h, a_dev, c_dev, nbands, q, nullptr, 0, stream);
+}
+
+int gh_lfc_integrate_ws(const gh_lfc* h, const void* a_dev, void* c_dev,
+                        int64_t nbands, int q, void* work_dev, int64_t work_bytes,
+                        void* stream) {
     GH_REQUIRE(h, GH_ERR_ARG, "lfc_integrate: null handle");
     GH_REQUIRE(nbands >= 0, GH_ERR_ARG, "lfc_integrate: nbands < 0");
     GH_REQUIRE(q >= 0 && (q < h->nq || (h->nq == 0 && q == 0)), GH_ERR_ARG,
@@ -698,17 +754,39 @@ int gh_lfc_integrate(const gh_lfc* h, const void* a_dev, void* c_dev,
     const int bt = h->dtype == GH_C128 ? IntBT<cplx<double>>::value
                    : h->dtype == GH_C64 ? IntBT<cplx<float>>::value
                                         : IntBT<double>::value;
-    dim3 grid(h->natoms, (unsigned)((nbands + bt - 1) / bt));
-    const void* ph = phase_table(h, q);
-#define ARGS(V, S) (const V*)a_dev, (V*)c_dev, h->entry_ptr, h->M_ptr, h->A_off, h->G_e, h->w_e, \
-                   (const S*)h->A, (const S*)ph, h->ngpts, h->Mmax, (int)nbands, (S)h->dv
-    switch (h->dtype) {
-        case GH_F64: hipLaunchKernelGGL((lfc_integrate_kernel<double, double>), grid, dim3(256), 0, st, ARGS(double, double)); break;
-        case GH_C128: hipLaunchKernelGGL((lfc_integrate_kernel<cplx<double>, double>), grid, dim3(256), 0, st, ARGS(cplx<double>, double)); break;
-        case GH_F32: hipLaunchKernelGGL((lfc_integrate_kernel<float, float>), grid, dim3(256), 0, st, ARGS(float, float)); break;
-        case GH_C64: hipLaunchKernelGGL((lfc_integrate_kernel<cplx<float>, float>), grid, dim3(256), 0, st, ARGS(cplx<float>, float)); break;
+    int ns = 1;
+    if (work_dev) {
+        GH_REQUIRE(work_bytes >= gh_lfc_integrate_work(h, nbands), GH_ERR_ARG,
+                   "lfc_integrate: workspace of %lld bytes, %lld needed", (long long)work_bytes,
+                   (long long)gh_lfc_integrate_work(h, nbands));
+        GH_REQUIRE(((uintptr_t)work_dev & 15u) == 0, GH_ERR_ARG,
+                   "lfc_integrate: workspace not 16-byte aligned");
+        ns = integrate_slices(h, nbands);
     }
-#undef ARGS
+    dim3 grid(h->natoms, (unsigned)((nbands + bt - 1) / bt), (unsigned)ns);
+    const void* ph = phase_table(h, q);
+    const int64_t total = nbands * h->Mmax;
+#define INT_LAUNCH(V, S)                                                                    \
+    do {                                                                                    \
+        using W = typename Wide<V>::type;                                                   \
+        hipLaunchKernelGGL((lfc_integrate_kernel<V, S>), grid, dim3(256), 0, st,            \
+                           (const V*)a_dev, (V*)c_dev, ns > 1 ? (W*)work_dev : (W*)nullptr, \
+                           h->entry_ptr, h->M_ptr, h->A_off, h->G_e, h->w_e,                \
+                           (const S*)h->A, (const S*)ph, h->ngpts, h->Mmax, (int)nbands,    \
+                           (S)h->dv);                                                       \
+        GH_CHECK_LAUNCH();                                                                  \
+        if (ns > 1 && total > 0)                                                            \
+            hipLaunchKernelGGL((lfc_slices_kernel<V>), dim3((unsigned)((total + 255) / 256)), \
+                               dim3(256), 0, st, (const W*)work_dev, (V*)c_dev, total, ns,  \
+                               (double)(S)h->dv);                                           \
+    } while (0)
+    switch (h->dtype) {
+        case GH_F64: INT_LAUNCH(double, double); break;
+        case GH_C128: INT_LAUNCH(cplx<double>, double); break;
+        case GH_F32: INT_LAUNCH(float, float); break;
+        case GH_C64: INT_LAUNCH(cplx<float>, float); break;
+    }
+#undef INT_LAUNCH
     GH_CHECK_LAUNCH();
     return GH_OK;
 }

@@ -247,8 +247,13 @@ class LocalizedFunctionsCollection:
         kq = self._kpoint(q)
         with Staged(a_xG, dtype=self.dtype) as a, \
                 Staged(c_xM, writeback=True, dtype=self.dtype) as c:
-            _lib.check(self._lib.gh_lfc_integrate(
+            nwork = self._lib.gh_lfc_integrate_work(self.handle, nb)
+            work = None
+            if nwork > 0:
+                work = torch.empty(nwork, dtype=torch.uint8, device='cuda')
+            _lib.check(self._lib.gh_lfc_integrate_ws(
                 self.handle, a.data_ptr(), c.data_ptr(), nb, kq,
+                work.data_ptr() if nwork > 0 else None, nwork,
                 stream_ptr()))
         return c_xM
 

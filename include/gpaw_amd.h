@@ -213,6 +213,16 @@ int64_t gh_spline_to_grid(int l, int nbins, double dr, const double* coefs,
 int gh_lfc_integrate(const gh_lfc* h, const void* a_dev, void* c_dev,
                      int64_t nbands, int q, void* stream);
 
+/* The same with a caller-owned device workspace of
+ * gh_lfc_integrate_work(h, nbands) bytes (16-byte aligned; 0: none needed),
+ * which lets few atoms x bands spread each atom's points over several
+ * workgroups; their FP64 sums are added in a fixed order.  work_dev may be
+ * null: then as gh_lfc_integrate. */
+int64_t gh_lfc_integrate_work(const gh_lfc* h, int64_t nbands);
+int gh_lfc_integrate_ws(const gh_lfc* h, const void* a_dev, void* c_dev,
+                        int64_t nbands, int q, void* work_dev,
+                        int64_t work_bytes, void* stream);
+
 /* a[x, G] += sum_M c[x, M] A_M(G) [* conj(phase_q)]  (LFC.add_gpu,
  * lfc.py:416-419).  One launch over the grid points of the spheres' union:
  * one read-modify-write per point, the contributions of several atoms (or

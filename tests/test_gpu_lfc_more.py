@@ -209,3 +209,34 @@ def test_points_add_equals_colour_add(monkeypatch, dtype, k_c, ls_a, h):
     b_q = dev(a.copy())
     lfc.add_M(b_q, coef)
     assert torch.equal(b_p, b_q)
+
+
+@pytest.mark.parametrize('dtype', [np.float64, np.complex128, np.float32,
+                                   np.complex64])
+@pytest.mark.parametrize('nb', [1, 17, 900])
+def test_integrate_slices(dtype, nb):
+    """The split of an atom's points over workgroups (few atoms x bands),
+    with an empty atom and atoms of different size, against the unsplit
+    form: FP64 sums in another order, so 1e-13 of the largest coefficient
+    (one rounding to FP32 for single-precision data: 1e-6)."""
+    from gpaw_amd import _lib
+    from gpaw_amd._arrays import stream_ptr
+    rng = np.random.default_rng(5)
+    N_c = (16, 18, 20)
+    kd = (np.array([[0.25, 0.1, 0.0]]) if np.dtype(dtype).kind == 'c'
+          else None)
+    lfc, oracle = build(rng, N_c, 0.25, [(0, 0, 1, 1), (), (1,)], dtype, kd)
+    a = dev(rand(rng, (nb,) + N_c, dtype))
+    c = lfc.integrate_M(a)
+    ref = torch.empty_like(c)
+    L = _lib.lib()
+    nwork = L.gh_lfc_integrate_work(lfc.handle, nb)
+    assert nwork > 0
+    _lib.check(L.gh_lfc_integrate(lfc.handle, a.data_ptr(), ref.data_ptr(),
+                                  nb, 0, stream_ptr()))
+    tol = 1e-13 if np.dtype(dtype).itemsize >= 8 and dtype != np.complex64 \
+        else 1e-6
+    assert relerr(host(c), host(ref)) < tol
+    rc = L.gh_lfc_integrate_ws(lfc.handle, a.data_ptr(), ref.data_ptr(), nb,
+                               0, a.data_ptr(), nwork - 1, stream_ptr())
+    assert rc == -1 and b'workspace' in L.gh_last_error()
