@@ -60,8 +60,7 @@ __device__ __forceinline__ void narrow(cplx<double> a, cplx<S>* o) {
 
 template <typename V> struct IntBT { static constexpr int value = 16; };
 template <> struct IntBT<cplx<double>> { static constexpr int value = 8; };
-// complex64 sums in complex128: 8 bands keep the LDS of T and the FP64
-// reduction buffer at 48 KB
+// complex64 sums in complex128: 8 bands keep the LDS at 32 KB
 template <> struct IntBT<cplx<float>> { static constexpr int value = 8; };
 
 // integrate: one 256-thread block per (atom, band tile).  Per chunk of 256
@@ -88,10 +87,9 @@ lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
                      int64_t ngpts, int Mmax, int nbands, S dv) {
     constexpr int BT = IntBT<V>::value;
     using W = typename Wide<V>::type;
-    constexpr bool kWide = sizeof(W) > sizeof(V);
-    __shared__ V T[BT][kIntChunk];
-    // reduction buffer: T itself when the sums have the storage type
-    __shared__ W Tw[kWide ? BT * kIntChunk : 1];
+    // staged values, and after the last chunk the groups' sums
+    __shared__ __align__(16) W Tw[BT * kIntChunk];
+    V (*T)[kIntChunk] = reinterpret_cast<V(*)[kIntChunk]>(Tw);
     const int atom = blockIdx.x;
     const int x0 = blockIdx.y * BT;
     const int M0 = M_ptr[atom];
@@ -146,8 +144,23 @@ lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
         __syncthreads();
         const int n = (int)min<int64_t>(kIntChunk, e1 - eb);
         if (live) {
-            for (int el = grp; el < n; el += ngrp) {
-                const S Am = Aa[(eb - e0 + el) * nm + m];
+            // four function values in flight: one at a time, their latency
+            // was most of a chunk's time (complex64, 32 atoms x 128 bands at
+            // 96^3: 160 -> 95 us; FP64, 64 x 256 at 112^3: 266 -> 257 us)
+            const S* __restrict__ Ac = Aa + (eb - e0) * nm + m;
+            int el = grp;
+            for (; el + 3 * ngrp < n; el += 4 * ngrp) {
+                S Am[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) Am[u] = Ac[(int64_t)(el + u * ngrp) * nm];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int b = 0; b < BT; b++)
+                        acc[b] = fma_rs(widen(Am[u]), widen(T[b][el + u * ngrp]), acc[b]);
+            }
+            for (; el < n; el += ngrp) {
+                const S Am = Ac[(int64_t)el * nm];
 #pragma unroll
                 for (int b = 0; b < BT; b++)
                     acc[b] = fma_rs(widen(Am), widen(T[b][el]), acc[b]);
@@ -156,7 +169,7 @@ lfc_integrate_kernel(const V* __restrict__ a, V* __restrict__ c,
     }
     // reduce over entry groups: R[g][b][m] reuses T
     __syncthreads();
-    W* Rb = kWide ? Tw : reinterpret_cast<W*>(&T[0][0]);
+    W* Rb = Tw;
     if (live) {
 #pragma unroll
         for (int b = 0; b < BT; b++) Rb[(grp * BT + b) * nm + m] = acc[b];
