@@ -20,6 +20,19 @@ int stencil_apply_full(const gh_stencil* h, const void* in, void* out,
                        double alpha, double gamma, const double* eps,
                        hipStream_t st);
 
+// A stencil along the grid axes for the LDS-free kernel (stencil_direct.hip):
+// grid, boundaries, radius and coefficients; rows / planes: tile (0: chosen)
+constexpr int kDirectMaxR = 6;
+struct DirectStencil {
+    int n[3], pbc[3], R;
+    double c0, cm[3][kDirectMaxR], cp[3][kDirectMaxR];
+    int rows, planes;
+};
+int stencil_direct(int dtype, const DirectStencil& h, const void* in, void* out,
+                   int64_t nbands, const double* phase_cd, const void* vt,
+                   const void* src, double beta, double alpha, double gamma,
+                   const double* eps, hipStream_t st);
+
 // out = alpha * T(in)
 int transformer_apply_scaled(const gh_transformer* h, const void* in,
                              void* out, int64_t nbands,

@@ -1458,6 +1458,25 @@ template <> struct RingPPT<cplx<double>> { static constexpr int value = 1; };
 template <> struct RingPPT<float> { static constexpr int value = 4; };
 template <> struct RingPPT<cplx<float>> { static constexpr int value = 2; };
 
+int launch_direct(const gh_stencil* h, const void* in, void* out, int64_t nb,
+                  const double* ph, const void* vt, const void* src, double beta,
+                  double al, double ga, const double* eps, hipStream_t st) {
+    DirectStencil d;
+    for (int c = 0; c < 3; c++) {
+        d.n[c] = (int)h->n[c];
+        d.pbc[c] = h->pbc[c];
+        for (int j = 0; j < kMaxR; j++) {
+            d.cm[c][j] = h->cm[c][j];
+            d.cp[c][j] = h->cp[c][j];
+        }
+    }
+    d.R = h->R;
+    d.c0 = h->c0;
+    d.rows = h->ty_req;
+    d.planes = h->lx_req;
+    return stencil_direct(h->dtype, d, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
+}
+
 template <typename V, typename S, int PPT>
 int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
                const double* ph, const void* vt, const void* src, double beta,
@@ -1486,6 +1505,13 @@ int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
             }
         }
         if (rc != GH_ERR_UNSUPPORTED) return rc;
+        // Few points: the register kernel below splits a grid along y only
+        // and leaves most CUs idle (191 x 191 x 223 FP64, one Jacobi sweep:
+        // 589 us on 22 blocks against 56 us); with enough bands to fill the
+        // GPU its LDS tile is the cheaper source of neighbours (48 bands of
+        // 95 x 95 x 103: 418 against 474 us).
+        const int64_t points = nb * h->n[0] * h->n[1] * h->n[2];
+        if (points <= 16 * 1024 * 1024) return launch_direct(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
     }
     switch (h->R) {
         case 1: return launch_cfd_r<V, S, 1, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
