@@ -7,18 +7,11 @@
 // the fly from the interior.
 //
 // Axis-aligned ("central finite difference") stencils -- every Laplace on an
-// orthorhombic cell -- use stencil_cfd_kernel:
-//   * a block owns one band, a tile of `ty` full (y, z) rows and a run of
-//     `lx` x-planes; it marches along x (the slowest axis);
-//   * each thread owns PPT points of the tile and keeps a register queue of
-//     the 2R+1 x-planes through them, so the x-neighbours cost no extra loads;
-//   * the current plane's tile plus R ghost rows above and below lives in
-//     LDS (double buffered, one barrier per plane); y- and z-neighbours are
-//     read from LDS, the z-wrap is an index wrap inside the LDS row;
-//   * each plane of the tile is a contiguous run of (ty + 2R) * n2 values in
-//     HBM, so every load is fully coalesced.
-// Other stencils (non-orthogonal cells) use stencil_generic_kernel, one
-// thread per point reading its neighbours through the cache hierarchy.
+// orthorhombic cell -- run in stencil_rows.hip (a ring of planes in LDS, for
+// all but small calls) or stencil_direct.hip (no LDS); the batched cells of
+// this file have a persistent ring kernel of their own.  Other stencils
+// (non-orthogonal cells) use stencil_generic_kernel, one thread per point
+// reading its neighbours through the cache hierarchy.
 #include <cstdarg>
 #include <cstdlib>
 #include <type_traits>
@@ -79,193 +72,9 @@ __device__ __forceinline__ V load_x(const V* __restrict__ inb, int x, int yz,
     return mul_phase(v, ph.re[0][d], ph.im[0][d]);
 }
 
-constexpr int kCfdMaxThreads = 512;
-
-// kGhostSlots: ghost values each thread prefetches per plane (1 when the
-// 2R ghost rows fit in one pass of the block, else 4 plus a tail loop).
-template <typename V, typename S, int R, int PPT, int kGhostSlots, bool HAS_V,
-          bool HAS_SRC>
-__global__ void __launch_bounds__(kCfdMaxThreads)
-stencil_cfd_kernel(const V* __restrict__ in, V* __restrict__ out,
-                   const S* __restrict__ vt, const V* __restrict__ src,
-                   S beta, CfdCoefs<S> cf, CfdGeom g, PhaseArgs<S> ph) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    V* lds = reinterpret_cast<V*>(smem_raw);
-
-    const int n2 = g.n2;
-    const int NT = blockDim.x;
-    const int tiles_per_band = g.nyt * g.nxc;
-    const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-    const int band = b / tiles_per_band;
-    const int rem = b - band * tiles_per_band;
-    const S c0b = cf.eps ? cf.c0 - (S)cf.eps[band] : cf.c0;
-    const int xc = rem / g.nyt;
-    const int yt = rem - xc * g.nyt;
-    const int y0 = yt * g.ty;
-    const int tye = min(g.ty, g.n1 - y0);
-    const int x0 = xc * g.lx;
-    const int x1 = min(x0 + g.lx, g.n0);
-    const size_t plane = (size_t)g.n1 * n2;
-    const size_t bstride = plane * g.n0;
-    const V* __restrict__ inb = in + band * bstride;
-    V* __restrict__ outb = out + band * bstride;
-    const V* __restrict__ srcb = HAS_SRC ? src + band * bstride : nullptr;
-    const int tile_pts = tye * n2;
-    const int bufsz = (g.ty + 2 * R) * n2;
-    const int nghost = 2 * R * n2;
-
-    // own points of this thread: tile index p = tid + k * NT
-    int yl[PPT], zz[PPT], yz[PPT];
-    bool act[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        int p = threadIdx.x + k * NT;
-        act[k] = p < tile_pts;
-        int pp = act[k] ? p : 0;
-        yl[k] = pp / n2;
-        zz[k] = pp - yl[k] * n2;
-        yz[k] = (y0 + yl[k]) * n2 + zz[k];
-    }
-    // ghost rows (R above, R below the tile): LDS slot, in-plane source
-    // offset and kind (0 interior, 1 wrapped low, 2 wrapped high, 3 zero)
-    int gl[kGhostSlots], gsrc[kGhostSlots], gkind[kGhostSlots];
-#pragma unroll
-    for (int i = 0; i < kGhostSlots; i++) {
-        int idx = threadIdx.x + i * NT;
-        gl[i] = -1;
-        gsrc[i] = 0;
-        gkind[i] = 3;
-        if (idx < nghost) {
-            int hr = idx / n2;
-            int z = idx - hr * n2;
-            int lrow = hr < R ? hr : hr + tye;
-            int y = y0 - R + lrow;
-            gl[i] = lrow * n2 + z;
-            if (y >= 0 && y < g.n1) { gkind[i] = 0; gsrc[i] = y * n2 + z; }
-            else if (g.pbc1) {
-                gkind[i] = y < 0 ? 1 : 2;
-                gsrc[i] = (y < 0 ? y + g.n1 : y - g.n1) * n2 + z;
-            }
-        }
-    }
-
-    auto ghost_value = [&](const V* __restrict__ pl, int src_off, int kind) {
-        if (kind == 0) return pl[src_off];
-        if (kind == 3) return vzero<V>();
-        V v = pl[src_off];
-        return kind == 1 ? mul_phase(v, ph.re[1][1], ph.im[1][1])
-                         : mul_phase(v, ph.re[1][0], ph.im[1][0]);
-    };
-
-    // register queue: q[k][j] holds plane (x - R + j) at own point k
-    V q[PPT][2 * R + 1];
-#pragma unroll
-    for (int j = 0; j < 2 * R; j++)
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-            q[k][j] = act[k] ? load_x(inb, x0 - R + j, yz[k], g, ph) : vzero<V>();
-
-    // Two-deep prefetch ring: slot s holds the own points of plane
-    // (x + R) and the ghost rows of plane x for the iteration that uses it;
-    // the loads for plane x + 2 are issued as soon as slot s is consumed, so
-    // two planes of loads are in flight behind each barrier.
-    V nq[2][PPT];
-    V ng[2][kGhostSlots];
-    auto prefetch = [&](int xn, V* nqs, V* ngs) {
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-            nqs[k] = act[k] ? load_x(inb, xn + R, yz[k], g, ph) : vzero<V>();
-        const V* pl = inb + (size_t)xn * plane;
-#pragma unroll
-        for (int i = 0; i < kGhostSlots; i++)
-            ngs[i] = gl[i] >= 0 ? ghost_value(pl, gsrc[i], gkind[i]) : vzero<V>();
-    };
-    prefetch(x0, nq[0], ng[0]);
-    if (x0 + 1 < x1) prefetch(x0 + 1, nq[1], ng[1]);
-
-    auto step = [&](int x, V* nqs, V* ngs) {
-        V* buf = lds + (x & 1) * bufsz;
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            q[k][2 * R] = nqs[k];
-            if (act[k]) buf[(yl[k] + R) * n2 + zz[k]] = q[k][R];
-        }
-#pragma unroll
-        for (int i = 0; i < kGhostSlots; i++)
-            if (gl[i] >= 0) buf[gl[i]] = ngs[i];
-        // ghosts beyond the prefetched slots (very small tiles only)
-        if (nghost > kGhostSlots * NT) {
-            const V* pl = inb + (size_t)x * plane;
-            for (int idx = threadIdx.x + kGhostSlots * NT; idx < nghost; idx += NT) {
-                int hr = idx / n2;
-                int z = idx - hr * n2;
-                int lrow = hr < R ? hr : hr + tye;
-                int y = y0 - R + lrow;
-                V v;
-                if (y >= 0 && y < g.n1) v = pl[y * n2 + z];
-                else if (g.pbc1) {
-                    int d = y < 0 ? 1 : 0;
-                    int yy = y < 0 ? y + g.n1 : y - g.n1;
-                    v = mul_phase(pl[yy * n2 + z], ph.re[1][d], ph.im[1][d]);
-                } else v = vzero<V>();
-                buf[lrow * n2 + z] = v;
-            }
-        }
-        if (x + 2 < x1) prefetch(x + 2, nqs, ngs);
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            if (!act[k]) continue;
-            const int row = yl[k] + R;
-            const int z = zz[k];
-            V acc = vscale(q[k][R], c0b);
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                acc = fma_rs(cf.cm[0][j], q[k][R - 1 - j], acc);
-                acc = fma_rs(cf.cp[0][j], q[k][R + 1 + j], acc);
-            }
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                acc = fma_rs(cf.cm[1][j], buf[(row - 1 - j) * n2 + z], acc);
-                acc = fma_rs(cf.cp[1][j], buf[(row + 1 + j) * n2 + z], acc);
-            }
-            const V* brow = buf + row * n2;
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                int zm = z - 1 - j;
-                V vm;
-                if (zm >= 0) vm = brow[zm];
-                else if (g.pbc2) vm = mul_phase(brow[zm + n2], ph.re[2][1], ph.im[2][1]);
-                else vm = vzero<V>();
-                int zp = z + 1 + j;
-                V vp;
-                if (zp < n2) vp = brow[zp];
-                else if (g.pbc2) vp = mul_phase(brow[zp - n2], ph.re[2][0], ph.im[2][0]);
-                else vp = vzero<V>();
-                acc = fma_rs(cf.cm[2][j], vm, acc);
-                acc = fma_rs(cf.cp[2][j], vp, acc);
-            }
-            const size_t gi = (size_t)x * plane + yz[k];
-            if (HAS_V) acc = fma_rs(vt[gi], q[k][R], acc);
-            if (HAS_SRC) acc = fma_rs(beta, srcb[gi], acc);
-            outb[gi] = acc;
-        }
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-#pragma unroll
-            for (int j = 0; j < 2 * R; j++) q[k][j] = q[k][j + 1];
-    };
-
-    for (int x = x0; x < x1; x += 2) {
-        step(x, nq[0], ng[0]);
-        if (x + 1 < x1) step(x + 1, nq[1], ng[1]);
-    }
-}
-
 // ------------------------------------------------- LDS-ring stencil --
-// The high-throughput form of stencil_cfd_kernel.  The block owns one band,
-// a tile of ty full (y, z) rows and a run of x-planes, as above, but plane
-// tiles (ty + 2R rows, ghosts included) are streamed HBM -> LDS by
+// The batched cells' form of the ring.  The block owns one band and a tile
+// of ty full (y, z) rows and marches along x; plane tiles (ty + 2R rows, ghosts included) are streamed HBM -> LDS by
 // global_load_lds DMA into a ring of P = R + D + 1 slots, D planes ahead of
 // use, by D loader wavefronts: loader w owns the planes xp with
 // (xp - x0) % D == w, so it has exactly one plane in flight and waits for it
@@ -295,11 +104,8 @@ struct RingGeom {
     int nload;            // loader wavefronts (= prefetch depth D)
     int ncomp;            // compute wavefronts
     int bgroup;           // bands per scheduling group
-    int nt_store;         // streaming stores of the output
     int nbands;
     int nlogical;         // logical tiles: nbands * nyt * nxc
-    int rounds;           // logical tiles per block (persistent launch)
-    int cplx_fast;        // complex data, trivial y / z Bloch phases
 };
 
 // Block -> (band, x chunk, y tile).  Logical ids of one XCD are contiguous
@@ -321,13 +127,6 @@ __device__ __forceinline__ void ring_block_coords(const RingGeom& rg, int L,
     xc = tile / rg.g.nyt;
     yt = tile - xc * rg.g.nyt;
 }
-
-// LDS layout of the ring kernel (in elements of V): P psi slots of
-// (ty + 2R) rows, then D + 1 slots of ty rows for the potential (as S) and
-// D + 1 slots of ty rows for src, when present.
-struct RingLayout {
-    int psi_slot;               // elements per slot
-};
 
 // SYM: the coefficients of +j and -j are equal along every axis (every
 // Laplacian); the paired real path then adds the two neighbours first and
@@ -540,8 +339,7 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                 if (HAS_SRC) acc = ss * beta + acc;
                 if (act) {
                     V4* o = reinterpret_cast<V4*>(outb + gi);
-                    if (rg.nt_store) __builtin_nontemporal_store(acc, o);
-                    else *o = acc;
+                    __builtin_nontemporal_store(acc, o);
                 }
 #pragma unroll
                 for (int j = 0; j < 2 * R; j++) q[j] = q[j + 1];
@@ -683,8 +481,7 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                 if (HAS_SRC) acc = ss * beta + acc;
                 if (act) {
                     V2* o = reinterpret_cast<V2*>(outb + gi);
-                    if (rg.nt_store) __builtin_nontemporal_store(acc, o);
-                    else *o = acc;
+                    __builtin_nontemporal_store(acc, o);
                 }
 #pragma unroll
                 for (int j = 0; j < 2 * R; j++) q[j] = q[j + 1];
@@ -693,276 +490,6 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
         if (g.pbc2) march(std::true_type{});
         else march(std::false_type{});
         return;
-    }
-    if constexpr (is_complex<V>::value && PPT == 2) {
-      {
-        // Complex data whose y and z Bloch phases are 1: the stencil's real
-        // coefficients act on real and imaginary parts alike, so this is the
-        // paired path above on (re, im) pairs -- a thread owns two
-        // z-adjacent points as one 4-vector (re0, im0, re1, im1).  Only the
-        // x-wrap phase (uniform per plane) is applied, at the queue refill.
-        typedef S V4 __attribute__((ext_vector_type(4)));
-        typedef S S2 __attribute__((ext_vector_type(2)));
-        const int np = n2 / 2;
-        const int pidx = threadIdx.x;
-        const bool act = pidx < tye * np;
-        const int pp = act ? pidx : 0;
-        const int yl = pp / np;
-        const int zp = pp - yl * np;
-        const int yz = (y0 + yl) * n2 + 2 * zp;
-        constexpr int NPW = (R + 1) / 2;
-        int zoff[2 * NPW];
-        bool zout[2 * NPW];
-#pragma unroll
-        for (int i = 0; i < NPW; i++) {
-            int zm = zp - 1 - i, zq = zp + 1 + i;
-            zout[i] = zm < 0 && !g.pbc2;
-            zout[NPW + i] = zq >= np && !g.pbc2;
-            zoff[i] = zm < 0 ? zm + np : zm;
-            zoff[NPW + i] = zq >= np ? zq - np : zq;
-        }
-        if (!g.pbc1) {
-            for (int r = 0; r < 2 * R; r++) {
-                const int lrow = r < R ? r : tye + r;
-                const int y = y0 - R + lrow;
-                if (y >= 0 && y < g.n1) continue;
-                for (int sl = 0; sl < P; sl++)
-                    for (int e = pidx; e < n2; e += rg.ncomp * 64)
-                        ring[sl * slot + lrow * n2 + e] = vzero<V>();
-            }
-        }
-        // (symmetric stencils only: with both signs pinned the register
-        // file overflows)
-        S k0 = c0b;
-        S km[3][R], kp[3][R];
-        if (SYM) asm volatile("" : "+v"(k0));
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                km[c][j] = cf.cm[c][j];
-                kp[c][j] = SYM ? km[c][j] : cf.cp[c][j];
-                if (SYM) asm volatile("" : "+v"(km[c][j]));
-            }
-        auto pack = [&](V a, V b) { return V4{a.re, a.im, b.re, b.im}; };
-        V4 q[2 * R + 1];
-#pragma unroll
-        for (int j = 0; j < 2 * R; j++)
-            q[j] = pack(load_x(inb, x0 - R + j, yz, g, ph),
-                        load_x(inb, x0 - R + j, yz + 1, g, ph));
-        const S pr = ph.re[0][0], pi = ph.im[0][0];   // x-wrap high -> low
-        for (int x = x0; x < x1; x++) {
-            ring_barrier();
-            {
-                const int xp = x + R;
-                const V4* sl = reinterpret_cast<const V4*>(ring + ((xp - x0) % P) * slot);
-                V4 v = sl[(yl + R) * np + zp];
-                if (xp >= g.n0) {
-                    if (!g.pbc0) v = V4{0, 0, 0, 0};
-                    else v = V4{v.x * pr - v.y * pi, v.x * pi + v.y * pr,
-                                v.z * pr - v.w * pi, v.z * pi + v.w * pr};
-                }
-                q[2 * R] = v;
-            }
-            const size_t gi = (size_t)x * plane + yz;
-            S2 vv;
-            V4 ss;
-            if (HAS_V) vv = *reinterpret_cast<const S2*>(vt + gi);
-            if (HAS_SRC) ss = *reinterpret_cast<const V4*>(src + band * bstride + gi);
-            const V4* sl = reinterpret_cast<const V4*>(ring + ((x - x0) % P) * slot);
-            V4 acc = q[R] * k0;
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                if constexpr (SYM) {
-                    acc = (q[R - 1 - j] + q[R + 1 + j]) * km[0][j] + acc;
-                } else {
-                    acc = q[R - 1 - j] * km[0][j] + acc;
-                    acc = q[R + 1 + j] * kp[0][j] + acc;
-                }
-            }
-            const int row = yl + R;
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                const V4 m = sl[(row - 1 - j) * np + zp];
-                const V4 pv = sl[(row + 1 + j) * np + zp];
-                if constexpr (SYM) {
-                    acc = (m + pv) * km[1][j] + acc;
-                } else {
-                    acc = m * km[1][j] + acc;
-                    acc = pv * kp[1][j] + acc;
-                }
-            }
-            V4 w[2 * NPW + 1];
-            w[NPW] = q[R];
-            const V4* brow = sl + row * np;
-#pragma unroll
-            for (int i = 0; i < NPW; i++) {
-                V4 lo = brow[zoff[i]], hi = brow[zoff[NPW + i]];
-                if (zout[i]) lo = V4{0, 0, 0, 0};
-                if (zout[NPW + i]) hi = V4{0, 0, 0, 0};
-                w[NPW - 1 - i] = lo;
-                w[NPW + 1 + i] = hi;
-            }
-            // complex element e of the window (pair e >> 1, point e & 1)
-            auto we = [&](int e) {
-                return (e & 1) ? S2{w[e >> 1].z, w[e >> 1].w} : S2{w[e >> 1].x, w[e >> 1].y};
-            };
-            S2 a0 = S2{acc.x, acc.y}, a1 = S2{acc.z, acc.w};
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                const int c = 2 * NPW;
-                if constexpr (SYM) {
-                    a0 = (we(c - 1 - j) + we(c + 1 + j)) * km[2][j] + a0;
-                    a1 = (we(c - j) + we(c + 2 + j)) * km[2][j] + a1;
-                } else {
-                    a0 = we(c - 1 - j) * km[2][j] + a0;
-                    a0 = we(c + 1 + j) * kp[2][j] + a0;
-                    a1 = we(c - j) * km[2][j] + a1;
-                    a1 = we(c + 2 + j) * kp[2][j] + a1;
-                }
-            }
-            acc = V4{a0.x, a0.y, a1.x, a1.y};
-            if (HAS_V) acc = V4{vv.x, vv.x, vv.y, vv.y} * q[R] + acc;
-            if (HAS_SRC) acc = ss * beta + acc;
-            if (act) {
-                V4* o = reinterpret_cast<V4*>(outb + gi);
-                if (rg.nt_store) __builtin_nontemporal_store(acc, o);
-                else *o = acc;
-            }
-#pragma unroll
-            for (int j = 0; j < 2 * R; j++) q[j] = q[j + 1];
-        }
-        return;
-      }
-    } else {
-    // general path: complex data with Bloch phases (one point per thread)
-    const int NT = rg.ncomp * 64;
-    const int tile_pts = tye * n2;
-    int yl[PPT], zz[PPT], yz[PPT];
-    bool act[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        int p = threadIdx.x + k * NT;
-        act[k] = p < tile_pts;
-        int pp = act[k] ? p : 0;
-        yl[k] = pp / n2;
-        zz[k] = pp - yl[k] * n2;
-        yz[k] = (y0 + yl[k]) * n2 + zz[k];
-    }
-    // y-ghost rows of the slot: R below (local rows 0..R-1) and R above
-    // (local rows R+tye..); kind per row offset j: 0 interior, 1 low wrap,
-    // 2 high wrap, 3 zero
-    auto row_kind = [&](int lrow) {
-        int y = y0 - R + lrow;
-        if (y >= 0 && y < g.n1) return 0;
-        if (!g.pbc1) return 3;
-        return y < 0 ? 1 : 2;
-    };
-    auto slot_val = [&](const V* sl, int lrow, int z) {
-        int kind = row_kind(lrow);
-        if (kind == 0) return sl[lrow * n2 + z];
-        if (kind == 3) return vzero<V>();
-        V v = sl[lrow * n2 + z];
-        return kind == 1 ? mul_phase(v, ph.re[1][1], ph.im[1][1])
-                         : mul_phase(v, ph.re[1][0], ph.im[1][0]);
-    };
-
-    V q[PPT][2 * R + 1];
-#pragma unroll
-    for (int j = 0; j < 2 * R; j++)
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-            q[k][j] = act[k] ? load_x(inb, x0 - R + j, yz[k], g, ph) : vzero<V>();
-    for (int x = x0; x < x1; x++) {
-        ring_barrier();
-        // queue refill: plane x + R (wrapped with phase, or zero)
-        {
-            const int xp = x + R;
-            const V* sl = ring + ((xp - x0) % P) * slot;
-            const bool wrap = xp >= g.n0;
-            const bool zero = wrap && !g.pbc0;
-#pragma unroll
-            for (int k = 0; k < PPT; k++) {
-                V v = sl[(yl[k] + R) * n2 + zz[k]];
-                if (zero) v = vzero<V>();
-                else if (wrap) v = mul_phase(v, ph.re[0][0], ph.im[0][0]);
-                q[k][2 * R] = act[k] ? v : vzero<V>();
-            }
-        }
-        // potential and src at the own points of plane x: plain loads
-        // (L2-resident for the potential), issued before the LDS work
-        S vv[PPT];
-        V ss[PPT];
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            const size_t gi = (size_t)x * plane + yz[k];
-            vv[k] = HAS_V ? vt[gi] : (S)0;
-            ss[k] = HAS_SRC ? src[band * bstride + gi] : vzero<V>();
-        }
-        const V* sl = ring + ((x - x0) % P) * slot;
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            if (!act[k]) continue;
-            const int row = yl[k] + R;
-            const int z = zz[k];
-            V acc = vscale(q[k][R], c0b);
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                acc = fma_rs(cf.cm[0][j], q[k][R - 1 - j], acc);
-                acc = fma_rs(cf.cp[0][j], q[k][R + 1 + j], acc);
-            }
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                acc = fma_rs(cf.cm[1][j], slot_val(sl, row - 1 - j, z), acc);
-                acc = fma_rs(cf.cp[1][j], slot_val(sl, row + 1 + j, z), acc);
-            }
-            const V* brow = sl + row * n2;
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                int zm = z - 1 - j;
-                V vm;
-                if (zm >= 0) vm = brow[zm];
-                else if (g.pbc2) vm = mul_phase(brow[zm + n2], ph.re[2][1], ph.im[2][1]);
-                else vm = vzero<V>();
-                int zp = z + 1 + j;
-                V vp;
-                if (zp < n2) vp = brow[zp];
-                else if (g.pbc2) vp = mul_phase(brow[zp - n2], ph.re[2][0], ph.im[2][0]);
-                else vp = vzero<V>();
-                acc = fma_rs(cf.cm[2][j], vm, acc);
-                acc = fma_rs(cf.cp[2][j], vp, acc);
-            }
-            if (HAS_V) acc = fma_rs(vv[k], q[k][R], acc);
-            if (HAS_SRC) acc = fma_rs(beta, ss[k], acc);
-            if (rg.nt_store) store_nt(outb + (size_t)x * plane + yz[k], acc);
-            else outb[(size_t)x * plane + yz[k]] = acc;
-        }
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-#pragma unroll
-            for (int j = 0; j < 2 * R; j++) q[k][j] = q[k][j + 1];
-    }
-    }  // general path
-}
-
-template <typename V, typename S, int R, int PPT, bool HAS_V, bool HAS_SRC,
-          bool SYM = false>
-__global__ void __launch_bounds__(kRingMaxThreads)
-stencil_ring_kernel(const V* __restrict__ in, V* __restrict__ out,
-                    const S* __restrict__ vt, const V* __restrict__ src,
-                    S beta, CfdCoefs<S> cf, RingGeom rg, PhaseArgs<S> ph,
-                    RingLayout lay) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    V* ring = reinterpret_cast<V*>(smem_raw);
-    const int Lbase = xcd_swizzle(blockIdx.x, gridDim.x);
-    // persistent blocks take logical tiles Lbase, Lbase + gridDim.x, ...;
-    // every wave of the block sees the same sequence
-    for (int rd = 0; rd < rg.rounds; rd++) {
-        const int L = Lbase + rd * (int)gridDim.x;
-        if (L >= rg.nlogical) break;
-        if (rd > 0) ring_barrier();   // last reads of the previous tile done
-        ring_tile<V, S, R, PPT, HAS_V, HAS_SRC, SYM>(in, out, vt, src, beta, cf, rg, ph, L,
-                                                      ring);
     }
 }
 
@@ -1149,123 +676,12 @@ struct gh_stencil {
     std::vector<double> coefs;
     std::vector<int64_t> offs;
     int ty_req = 0, lx_req = 0, depth_req = 0;
-    int bgroup_req = 0;      // bands per scheduling group (GPAW_AMD_BGROUP)
-    bool reg_only = false;   // GPAW_AMD_STENCIL=reg selects the register kernel
-    int persist = 0;         // persistent ring launch: 1 one block per CU,
-                             // n >= 8 a grid of n blocks (GPAW_AMD_PERSIST)
+    int mode = 0;            // GPAW_AMD_STENCIL: 1 reg (the kernel without LDS), 2 rows
 };
 
 using namespace gh;
 
-namespace {
-
-template <typename S>
-PhaseArgs<S> phase_args(const double* phase_cd) {
-    Phases p = make_phases(phase_cd);
-    PhaseArgs<S> a;
-    for (int c = 0; c < 3; c++)
-        for (int d = 0; d < 2; d++) {
-            a.re[c][d] = (S)p.re[c][d];
-            a.im[c][d] = (S)p.im[c][d];
-        }
-    return a;
-}
-
-struct TileChoice {
-    int ty, lx, ppt, threads;
-    size_t lds;
-};
-
-TileChoice choose_tile(const gh_stencil* h, int vsize, int ppt) {
-    const int n1 = (int)h->n[1], n2 = (int)h->n[2], n0 = (int)h->n[0];
-    const int R = h->R;
-    const size_t lds_cap = 64 * 1024;
-    TileChoice t{};
-    t.ppt = ppt;
-    int ty = h->ty_req > 0 ? h->ty_req : 0;
-    if (ty == 0) {
-        // largest divisor-friendly row count that fits the LDS and 1024
-        // threads; prefer divisors of n1 to avoid a ragged last tile
-        int best = 1;
-        for (int c = 1; c <= n1; c++) {
-            size_t lds = 2 * (size_t)(c + 2 * R) * n2 * vsize;
-            int thr = (c * n2 + ppt - 1) / ppt;
-            if (lds > lds_cap || thr > kCfdMaxThreads) break;
-            if (n1 % c == 0 || c == n1) best = c;
-        }
-        ty = best;
-        // ragged tiles are fine if no divisor >= 8 exists
-        if (ty < 8) {
-            for (int c = n1; c >= 1; c--) {
-                size_t lds = 2 * (size_t)(c + 2 * R) * n2 * vsize;
-                int thr = (c * n2 + ppt - 1) / ppt;
-                if (lds <= lds_cap && thr <= kCfdMaxThreads) { ty = c; break; }
-            }
-        }
-    }
-    ty = std::min(ty, n1);
-    t.ty = ty;
-    t.lx = h->lx_req > 0 ? std::min<int>(h->lx_req, n0) : n0;
-    int thr = (ty * n2 + ppt - 1) / ppt;
-    t.threads = ((thr + 63) / 64) * 64;
-    t.lds = 2 * (size_t)(ty + 2 * R) * n2 * vsize;
-    return t;
-}
-
-template <typename V, typename S, int R, int PPT>
-int launch_cfd_r(const gh_stencil* h, const void* in, void* out,
-                 int64_t nbands, const double* phase_cd, const void* vt,
-                 const void* src, double beta, double alpha, double gamma,
-                 const double* eps, hipStream_t st) {
-    TileChoice t = choose_tile(h, sizeof(V), PPT);
-    GH_REQUIRE(t.threads <= kCfdMaxThreads && t.lds <= 64 * 1024, GH_ERR_UNSUPPORTED,
-               "stencil: grid rows of %lld points do not fit one block",
-               (long long)h->n[2]);
-    CfdGeom g;
-    g.n0 = (int)h->n[0]; g.n1 = (int)h->n[1]; g.n2 = (int)h->n[2];
-    g.pbc0 = h->pbc[0]; g.pbc1 = h->pbc[1]; g.pbc2 = h->pbc[2];
-    g.ty = t.ty; g.lx = t.lx;
-    g.nyt = (g.n1 + t.ty - 1) / t.ty;
-    g.nxc = (g.n0 + t.lx - 1) / t.lx;
-    CfdCoefs<S> cf;
-    cf.c0 = (S)(alpha * h->c0 + gamma);
-    cf.eps = eps;
-    for (int c = 0; c < 3; c++)
-        for (int j = 0; j < kMaxR; j++) {
-            cf.cm[c][j] = (S)(alpha * h->cm[c][j]);
-            cf.cp[c][j] = (S)(alpha * h->cp[c][j]);
-        }
-    PhaseArgs<S> ph = phase_args<S>(phase_cd);
-    int64_t nblocks = nbands * (int64_t)g.nyt * g.nxc;
-    GH_REQUIRE(nblocks < (1ll << 31), GH_ERR_SHAPE, "stencil: too many blocks");
-    dim3 grid((unsigned)nblocks), block(t.threads);
-    const S* vtp = (const S*)vt;
-    const V* srcp = (const V*)src;
-    const bool gs1 = 2 * R * g.n2 <= t.threads;
-#define GH_LAUNCH_CFD(GS, HV, HS)                                              \
-    hipLaunchKernelGGL((stencil_cfd_kernel<V, S, R, PPT, GS, HV, HS>), grid,   \
-                       block, t.lds, st, (const V*)in, (V*)out, vtp, srcp,     \
-                       (S)beta, cf, g, ph)
-    if (gs1) {
-        if (vt && src) GH_LAUNCH_CFD(1, true, true);
-        else if (vt) GH_LAUNCH_CFD(1, true, false);
-        else if (src) GH_LAUNCH_CFD(1, false, true);
-        else GH_LAUNCH_CFD(1, false, false);
-    } else {
-        if (vt && src) GH_LAUNCH_CFD(4, true, true);
-        else if (vt) GH_LAUNCH_CFD(4, true, false);
-        else if (src) GH_LAUNCH_CFD(4, false, true);
-        else GH_LAUNCH_CFD(4, false, false);
-    }
-#undef GH_LAUNCH_CFD
-    GH_CHECK_LAUNCH();
-    return GH_OK;
-}
-
-// LDS-ring launch: returns GH_ERR_UNSUPPORTED when the shape does not fit
-// (rows not 16-byte multiples, or no tile fits the LDS), so the caller can
-// fall back to the register kernel.
-constexpr size_t kLdsBytes = 160 * 1024;
+namespace gh {
 
 // Compute units of the current device (queried once per device).
 int device_cu_count(int* out) {
@@ -1282,8 +698,8 @@ int device_cu_count(int* out) {
 
 // Raise a kernel's dynamic LDS limit to the whole 160 KB once per process
 // (not per launch).
-std::mutex g_attr_mutex;
-std::vector<const void*> g_attr_done;
+static std::mutex g_attr_mutex;
+static std::vector<const void*> g_attr_done;
 
 int ensure_max_lds(const void* fn, int bytes) {
     std::lock_guard<std::mutex> lock(g_attr_mutex);
@@ -1294,173 +710,32 @@ int ensure_max_lds(const void* fn, int bytes) {
     return GH_OK;
 }
 
-template <typename V, typename S, int R, int PPT>
-int launch_ring_r(const gh_stencil* h, const void* in, void* out,
-                  int64_t nbands, const double* phase_cd, const void* vt,
-                  const void* src, double beta, double alpha, double gamma,
-                  const double* eps, hipStream_t st) {
-    const int n0 = (int)h->n[0], n1 = (int)h->n[1], n2 = (int)h->n[2];
-    const int vs = (int)sizeof(V);
-    if ((n2 * vs) % kDmaBytes != 0) return GH_ERR_UNSUPPORTED;
-    // the plane DMA and the paired loads / stores move 16-byte vectors: a
-    // pointer off that alignment (a view at an odd element offset) takes the
-    // register kernel instead
-    auto aligned16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
-    if (!aligned16(in) || !aligned16(out) || (vt && !aligned16(vt)) ||
-        (src && !aligned16(src)))
-        return GH_ERR_UNSUPPORTED;
-    auto lds_of = [&](int c, int d) {
-        return (size_t)(R + d + 1) * (c + 2 * R) * n2 * vs;
-    };
-    // Largest tile (rows) that fits for each prefetch depth.  Explicit
-    // rows/depth (autotuner) override the automatic choice.
-    auto max_rows = [&](int d) {
-        int best = 0;
-        for (int c = 1; c <= n1; c++) {
-            int thr = (c * n2 + PPT - 1) / PPT;
-            int ncomp = (thr + 63) / 64;
-            if (lds_of(c, d) > kLdsBytes - 1024 || (ncomp + d) * 64 > kRingMaxThreads) break;
-            best = c;
-        }
-        return best;
-    };
-    auto divisor_rows = [&](int c) {   // prefer a divisor of n1 >= c / 2
-        for (int t = c; t >= std::max(1, c / 2); t--)
-            if (n1 % t == 0) return t;
-        return c;
-    };
-    int ty = 0, D = 0;
-    if (h->depth_req >= 2) {
-        D = h->depth_req;
-        int mr = max_rows(D);
-        ty = h->ty_req > 0 ? std::min(h->ty_req, mr) : divisor_rows(mr);
-    } else {
-        // depth 2 with the largest tile: measured faster than depth 3 with
-        // fewer rows (256 x 112^3 FP64: 16 rows x 2 planes 1.84 ms,
-        // 14 rows x 3 planes 1.96 ms)
-        D = 2;
-        ty = h->ty_req > 0 ? std::min(h->ty_req, max_rows(D)) : divisor_rows(max_rows(D));
-    }
-    if (ty <= 0) return GH_ERR_UNSUPPORTED;
-    const size_t lds = lds_of(ty, D);
-    RingLayout lay;
-    lay.psi_slot = (ty + 2 * R) * n2;
-    RingGeom rg;
-    CfdGeom& g = rg.g;
-    g.n0 = n0; g.n1 = n1; g.n2 = n2;
-    g.pbc0 = h->pbc[0]; g.pbc1 = h->pbc[1]; g.pbc2 = h->pbc[2];
-    g.ty = ty;
-    g.nyt = (n1 + ty - 1) / ty;
-    if (h->lx_req > 0) {
-        g.lx = std::min(h->lx_req, n0);
-    } else {
-        // one block per CU: when the bands x y-tiles do not cover the CUs,
-        // split the x-march into chunks (each chunk re-reads 2R planes),
-        // keeping chunks at least 4R planes long
-        int ncu = 0;
-        int rc = device_cu_count(&ncu);
-        if (rc != GH_OK) return rc;
-        const int64_t base = nbands * (int64_t)g.nyt;
-        int nxc = 1;
-        while (base * nxc < ncu && (n0 + nxc) / (nxc + 1) >= 4 * R) nxc++;
-        g.lx = (n0 + nxc - 1) / nxc;
-    }
-    g.nxc = (n0 + g.lx - 1) / g.lx;
-    rg.nload = D;
-    rg.ncomp = ((ty * n2 + PPT - 1) / PPT + 63) / 64;
-    rg.nbands = (int)nbands;
-    const int tiles = g.nyt * g.nxc;
-    const int64_t nlogical = nbands * (int64_t)tiles;
-    GH_REQUIRE(nlogical < (1ll << 31), GH_ERR_SHAPE, "stencil: too many blocks");
-    rg.nlogical = (int)nlogical;
-    rg.rounds = 1;
-    int64_t nblocks = nlogical;
-    int per_xcd = 32;                     // blocks running together per XCD
-    if (h->persist) {
-        // one resident block per CU walks its XCD's tiles band group by band
-        // group, so all blocks of an XCD stay on the same planes
-        int64_t n = h->persist;
-        if (n < kNumXCD) {
-            int ncu = 0;
-            int rc = device_cu_count(&ncu);
-            if (rc != GH_OK) return rc;
-            const int per_cu = std::max<int>(1, (int)(kLdsBytes / std::max<size_t>(lds, 1)));
-            n = (int64_t)ncu * per_cu;
-        }
-        n -= n % kNumXCD;
-        if (n >= kNumXCD && n < nlogical) {
-            nblocks = n;
-            rg.rounds = (int)((nlogical + n - 1) / n);
-            per_xcd = (int)(n / kNumXCD);
-        }
-    }
-    {
-        int bgr = h->bgroup_req > 0 ? h->bgroup_req : std::max(1, per_xcd / tiles);
-        rg.bgroup = std::min<int>(bgr, (int)nbands);
-        const char* nt = getenv("GPAW_AMD_NTSTORE");
-        rg.nt_store = nt ? atoi(nt) : 1;
-    }
-    CfdCoefs<S> cf;
-    cf.c0 = (S)(alpha * h->c0 + gamma);
-    cf.eps = eps;
+}  // namespace gh
+
+namespace {
+
+template <typename S>
+PhaseArgs<S> phase_args(const double* phase_cd) {
+    Phases p = make_phases(phase_cd);
+    PhaseArgs<S> a;
     for (int c = 0; c < 3; c++)
-        for (int j = 0; j < kMaxR; j++) {
-            cf.cm[c][j] = (S)(alpha * h->cm[c][j]);
-            cf.cp[c][j] = (S)(alpha * h->cp[c][j]);
+        for (int d = 0; d < 2; d++) {
+            a.re[c][d] = (S)p.re[c][d];
+            a.im[c][d] = (S)p.im[c][d];
         }
-    PhaseArgs<S> ph = phase_args<S>(phase_cd);
-    rg.cplx_fast = 0;
-    if (is_complex<V>::value) {
-        bool triv = true;
-        for (int c = 1; c < 3; c++)
-            for (int d = 0; d < 2; d++)
-                triv = triv && ph.re[c][d] == (S)1 && ph.im[c][d] == (S)0;
-        rg.cplx_fast = triv ? 1 : 0;
-    }
-    dim3 grid((unsigned)nblocks), block((rg.ncomp + rg.nload) * 64);
-    const S* vtp = (const S*)vt;
-    const V* srcp = (const V*)src;
-    // symmetric coefficients: the paired real path keeps half of them live
-    bool sym = true;
-    for (int c = 0; c < 3; c++)
-        for (int j = 0; j < R; j++) sym = sym && h->cm[c][j] == h->cp[c][j];
-    constexpr bool kPaired = PPT == 2 || PPT == 4;   // the vector paths take SYM
-#define GH_LAUNCH_RING_S(HV, HS, SY)                                           \
-    do {                                                                       \
-        auto kfn = stencil_ring_kernel<V, S, R, PPT, HV, HS, SY>;              \
-        int arc = ensure_max_lds((const void*)kfn, (int)kLdsBytes);            \
-        if (arc != GH_OK) return arc;                                          \
-        hipLaunchKernelGGL(kfn, grid, block, lds, st, (const V*)in, (V*)out,   \
-                           vtp, srcp, (S)beta, cf, rg, ph, lay);               \
-    } while (0)
-#define GH_LAUNCH_RING(HV, HS)                                                 \
-    do {                                                                       \
-        if constexpr (kPaired) {                                               \
-            if (sym) GH_LAUNCH_RING_S(HV, HS, true);                           \
-            else GH_LAUNCH_RING_S(HV, HS, false);                              \
-        } else {                                                               \
-            GH_LAUNCH_RING_S(HV, HS, false);                                   \
-        }                                                                      \
-    } while (0)
-    if (vt && src) GH_LAUNCH_RING(true, true);
-    else if (vt) GH_LAUNCH_RING(true, false);
-    else if (src) GH_LAUNCH_RING(false, true);
-    else GH_LAUNCH_RING(false, false);
-#undef GH_LAUNCH_RING
-#undef GH_LAUNCH_RING_S
-    GH_CHECK_LAUNCH();
-    return GH_OK;
+    return a;
 }
+
+constexpr size_t kLdsBytes = 160 * 1024;
 
 // points per compute thread of the ring kernel
 template <typename V> struct RingPPT { static constexpr int value = 2; };
-template <> struct RingPPT<cplx<double>> { static constexpr int value = 1; };
 template <> struct RingPPT<float> { static constexpr int value = 4; };
-template <> struct RingPPT<cplx<float>> { static constexpr int value = 2; };
 
-int launch_direct(const gh_stencil* h, const void* in, void* out, int64_t nb,
-                  const double* ph, const void* vt, const void* src, double beta,
-                  double al, double ga, const double* eps, hipStream_t st) {
+template <typename V, typename S>
+int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
+               const double* ph, const void* vt, const void* src, double beta,
+               double al, double ga, const double* eps, hipStream_t st) {
     DirectStencil d;
     for (int c = 0; c < 3; c++) {
         d.n[c] = (int)h->n[c];
@@ -1474,55 +749,19 @@ int launch_direct(const gh_stencil* h, const void* in, void* out, int64_t nb,
     d.c0 = h->c0;
     d.rows = h->ty_req;
     d.planes = h->lx_req;
-    return stencil_direct(h->dtype, d, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-}
-
-template <typename V, typename S, int PPT>
-int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
-               const double* ph, const void* vt, const void* src, double beta,
-               double al, double ga, const double* eps, hipStream_t st) {
-    if (!h->reg_only) {
-        constexpr int RP = RingPPT<V>::value;
-        int rc = GH_ERR_UNSUPPORTED;
-        // complex data takes the two-point path only when the y and z Bloch
-        // phases are 1; otherwise the one-point path with phases
-        bool two = RP > 1;
-        if (is_complex<V>::value && ph)
-            for (int c = 1; c < 3; c++)
-                for (int d = 0; d < 2; d++)
-                    two = two && ph[(c * 2 + d) * 2] == 1.0 && ph[(c * 2 + d) * 2 + 1] == 0.0;
-        if (two) {
-            switch (h->R) {
-                case 1: rc = launch_ring_r<V, S, 1, RP>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-                case 2: rc = launch_ring_r<V, S, 2, RP>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-                case 3: rc = launch_ring_r<V, S, 3, RP>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-            }
-        } else {
-            switch (h->R) {
-                case 1: rc = launch_ring_r<V, S, 1, 1>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-                case 2: rc = launch_ring_r<V, S, 2, 1>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-                case 3: rc = launch_ring_r<V, S, 3, 1>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st); break;
-            }
-        }
+    // The LDS ring needs a few MB to fill the GPU with its large blocks; up to
+    // 5 MB the kernel without LDS, split as finely as it likes, is faster:
+    // FP64, R = 3, 2 x 64^3 (4.2 MB) 7.3 against 8.6 us, 96^3 (7.1 MB) 9.8
+    // against 8.6, 64 x 24^3 (7.1 MB) 10.9 against 8.1.
+    const int64_t bytes = nb * h->n[0] * h->n[1] * h->n[2] * (int64_t)sizeof(V);
+    if (h->mode == 2 || (h->mode == 0 && bytes > 5 * 1024 * 1024)) {
+        int ncu = 0;
+        int rc = device_cu_count(&ncu);
+        if (rc != GH_OK) return rc;
+        rc = stencil_rows(h->dtype, d, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
         if (rc != GH_ERR_UNSUPPORTED) return rc;
-        // Few points: the register kernel below splits a grid along y only
-        // and leaves most CUs idle (191 x 191 x 223 FP64, one Jacobi sweep:
-        // 589 us on 22 blocks against 56 us); with enough bands to fill the
-        // GPU its LDS tile is the cheaper source of neighbours (48 bands of
-        // 95 x 95 x 103: 418 against 474 us).
-        const int64_t points = nb * h->n[0] * h->n[1] * h->n[2];
-        if (points <= 16 * 1024 * 1024) return launch_direct(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
     }
-    switch (h->R) {
-        case 1: return launch_cfd_r<V, S, 1, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-        case 2: return launch_cfd_r<V, S, 2, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-        case 3: return launch_cfd_r<V, S, 3, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-        case 4: return launch_cfd_r<V, S, 4, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-        case 5: return launch_cfd_r<V, S, 5, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-        case 6: return launch_cfd_r<V, S, 6, PPT>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
-    }
-    set_error("stencil: radius %d unsupported", h->R);
-    return GH_ERR_UNSUPPORTED;
+    return stencil_direct(h->dtype, d, in, out, nb, ph, vt, src, beta, al, ga, eps, st);
 }
 
 template <typename V, typename S>
@@ -1621,9 +860,6 @@ int plan_batch(BatchPlan& bp, const gh_stencil* const* ops, const int64_t* nband
         rc.rg.ncomp = ((ty * n2 + PPT - 1) / PPT + 63) / 64;
         rc.rg.nbands = (int)nbands[c];
         rc.rg.nlogical = (int)(nbands[c] * g.nyt);
-        rc.rg.rounds = 1;
-        rc.rg.nt_store = 1;
-        rc.rg.cplx_fast = 0;
         rc.cf.c0 = (S)h->c0;
         rc.cf.eps = nullptr;
         for (int a = 0; a < 3; a++)
@@ -1747,11 +983,7 @@ int gh_stencil_create(gh_stencil** out, int ncoefs, const double* coefs,
     h->coefs.assign(coefs, coefs + ncoefs);
     {
         const char* e = getenv("GPAW_AMD_STENCIL");
-        h->reg_only = e && std::string(e) == "reg";
-        const char* bg = getenv("GPAW_AMD_BGROUP");
-        h->bgroup_req = bg ? atoi(bg) : 0;
-        const char* pe = getenv("GPAW_AMD_PERSIST");
-        h->persist = pe ? std::max(0, atoi(pe)) : 0;
+        h->mode = !e ? 0 : std::string(e) == "reg" ? 1 : std::string(e) == "rows" ? 2 : 0;
     }
     h->offs.assign(offsets_pc, offsets_pc + 3 * ncoefs);
     h->R = 0;
@@ -2024,10 +1256,10 @@ int stencil_apply_full(const gh_stencil* h, const void* in_dev, void* out_dev,
     GH_REQUIRE(in_dev != out_dev, GH_ERR_ARG, "stencil_apply: in and out must differ");
     if (h->cfd) {
         switch (h->dtype) {
-            case GH_F64: return launch_cfd<double, double, 4>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
-            case GH_C128: return launch_cfd<cplx<double>, double, 2>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
-            case GH_F32: return launch_cfd<float, float, 8>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
-            case GH_C64: return launch_cfd<cplx<float>, float, 4>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_F64: return launch_cfd<double, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_C128: return launch_cfd<cplx<double>, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_F32: return launch_cfd<float, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_C64: return launch_cfd<cplx<float>, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
         }
     } else {
         GH_REQUIRE(!eps, GH_ERR_UNSUPPORTED,

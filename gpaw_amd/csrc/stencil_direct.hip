@@ -15,6 +15,7 @@
 // When PT does not divide n2 the last thread of a row is moved down to end
 // at the row's end and stores only the points that no other thread owns.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "internal.h"
@@ -42,7 +43,9 @@ __device__ __forceinline__ void load_n(const V* __restrict__ p, V* v) {
     __builtin_memcpy(v, p, N * sizeof(V));
 }
 
-template <typename V, typename S, int R, int PT, bool HAS_V, bool HAS_SRC>
+// SYM: equal coefficients at +j and -j; the sums then have the order of the
+// ring kernels, so a grid gives the same bits whichever kernel takes it.
+template <typename V, typename S, int R, int PT, bool SYM, bool HAS_V, bool HAS_SRC>
 __global__ void __launch_bounds__(512)
 stencil_direct_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __restrict__ vt,
                       const V* src, S beta, DirectArgs<S, R> g) {
@@ -161,25 +164,20 @@ stencil_direct_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __
 #pragma unroll
         for (int i = 0; i < PT; i++) {
             V a = vscale(q[R].v[i], c0b);
+            auto add_pair = [&](int c, int j, V m, V p) {
+                if constexpr (SYM) a = fma_rs(g.cm[c][j], vadd(m, p), a);
+                else a = fma_rs(g.cp[c][j], p, fma_rs(g.cm[c][j], m, a));
+            };
 #pragma unroll
-            for (int j = 0; j < R; j++) {
-                a = fma_rs(g.cm[0][j], q[R - 1 - j].v[i], a);
-                a = fma_rs(g.cp[0][j], q[R + 1 + j].v[i], a);
-            }
+            for (int j = 0; j < R; j++) add_pair(0, j, q[R - 1 - j].v[i], q[R + 1 + j].v[i]);
 #pragma unroll
-            for (int j = 0; j < R; j++) {
-                a = fma_rs(g.cm[1][j], yv[j].v[i], a);
-                a = fma_rs(g.cp[1][j], yv[R + j].v[i], a);
-            }
+            for (int j = 0; j < R; j++) add_pair(1, j, yv[j].v[i], yv[R + j].v[i]);
             // element e of the window z - R .. z + PT - 1 + R
             auto we = [&](int e) {
                 return e < R ? w[e] : e < R + PT ? q[R].v[e - R] : w[e - PT];
             };
 #pragma unroll
-            for (int j = 0; j < R; j++) {
-                a = fma_rs(g.cm[2][j], we(R + i - 1 - j), a);
-                a = fma_rs(g.cp[2][j], we(R + i + 1 + j), a);
-            }
+            for (int j = 0; j < R; j++) add_pair(2, j, we(R + i - 1 - j), we(R + i + 1 + j));
             if (HAS_V) a = fma_rs(vv[i], q[R].v[i], a);
             if (HAS_SRC) a = fma_rs(beta, sv.v[i], a);
             acc.v[i] = a;
@@ -250,15 +248,23 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
     g.nxc = (g.n0 + g.lx - 1) / g.lx;
     const int64_t nblocks = nbands * (int64_t)g.nyt * g.nzt * g.nxc;
     GH_REQUIRE(nblocks < (1ll << 31), GH_ERR_SHAPE, "stencil: too many blocks");
-#define GH_DIRECT(HV, HS)                                                                  \
-    hipLaunchKernelGGL((stencil_direct_kernel<V, S, R, PT, HV, HS>), dim3((unsigned)nblocks),  \
-                       dim3(threads), 0, st, (const V*)in, (V*)out, (const S*)vt,          \
-                       (const V*)src, (S)beta, g)
-    if (vt && src) GH_DIRECT(true, true);
-    else if (vt) GH_DIRECT(true, false);
-    else if (src) GH_DIRECT(false, true);
-    else GH_DIRECT(false, false);
+    bool sym = true;
+    for (int c = 0; c < 3; c++)
+        for (int j = 0; j < R; j++) sym = sym && h.cm[c][j] == h.cp[c][j];
+    auto go = [&](auto symmetric) {
+        constexpr bool SY = decltype(symmetric)::value;
+#define GH_DIRECT(HV, HS)                                                                     \
+    hipLaunchKernelGGL((stencil_direct_kernel<V, S, R, PT, SY, HV, HS>),                      \
+                       dim3((unsigned)nblocks), dim3(threads), 0, st, (const V*)in, (V*)out,  \
+                       (const S*)vt, (const V*)src, (S)beta, g)
+        if (vt && src) GH_DIRECT(true, true);
+        else if (vt) GH_DIRECT(true, false);
+        else if (src) GH_DIRECT(false, true);
+        else GH_DIRECT(false, false);
 #undef GH_DIRECT
+    };
+    if (sym) go(std::true_type{});
+    else go(std::false_type{});
     GH_CHECK_LAUNCH();
     return GH_OK;
 }

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 if not torch.cuda.is_available():
     pytest.skip('no GPU', allow_module_level=True)
 
-from gpaw_amd.fd_operators import Laplace  # noqa: E402
+from gpaw_amd.fd_operators import FDOperator, Laplace  # noqa: E402
 from gpaw_amd.grid_descriptor import GridDescriptor  # noqa: E402
 from oracle import grid as og  # noqa: E402
 from oracle import stencil as ost  # noqa: E402
@@ -51,8 +51,10 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize('kernel', ['', 'rows', 'reg'])
 @pytest.mark.parametrize('N_c,pbc,nb,n,dtype,k_c', CASES)
-def test_rows(N_c, pbc, nb, n, dtype, k_c):
+def test_rows(monkeypatch, N_c, pbc, nb, n, dtype, k_c, kernel):
+    monkeypatch.setenv('GPAW_AMD_STENCIL', kernel)
     rng = np.random.default_rng(3)
     N_c = np.array(N_c)
     gd = GridDescriptor(N_c, N_c * 0.4, pbc)
@@ -93,14 +95,21 @@ def test_rows(N_c, pbc, nb, n, dtype, k_c):
         check(sd, ref + 2.0 * src[pick])
         op.apply_shifted(ad, out, eps, ph, vt_g=vd)
         check(out, ref + (vt - eps[pick][:, None, None, None]) * a[pick])
+    for tile in ((1, 0), (3, 2), (0, 5)):
+        op.set_tile(*tile)
+        op.apply(ad, out, ph)
+        check(out, ref)
 
 
+@pytest.mark.parametrize('kernel', ['', 'rows', 'reg'])
 @pytest.mark.parametrize('value', [np.inf, -np.inf, np.nan])
 @pytest.mark.parametrize('N_c', [(9, 10, 12), (9, 10, 11)])
-def test_zero_boundary_keeps_infinities_apart(N_c, value):
+def test_zero_boundary_keeps_infinities_apart(monkeypatch, N_c, value,
+                                              kernel):
     """A point beyond a zero boundary contributes zero, not 0 * (a value of
     the grid): an infinity at a face reaches only the points whose stencil
     holds it."""
+    monkeypatch.setenv('GPAW_AMD_STENCIL', kernel)
     N_c = np.array(N_c)
     gd = GridDescriptor(N_c, N_c * 0.4, False)
     a = np.ones((1,) + tuple(gd.n_c))
@@ -113,3 +122,37 @@ def test_zero_boundary_keeps_infinities_apart(N_c, value):
     want = np.zeros(tuple(gd.n_c), bool)
     want[:4, 0, 0] = want[0, :4, 0] = want[0, 0, :4] = True
     assert (bad == want).all()
+
+
+@pytest.mark.parametrize('kernel', ['', 'rows', 'reg'])
+@pytest.mark.parametrize('N_c,pbc,nb,dtype,k_c', [
+    ((10, 12, 14), True, 2, np.float64, None),
+    ((64, 60, 53), False, 30, np.float64, None),
+    ((64, 60, 52), True, 30, np.float32, None),
+    ((40, 48, 45), True, 40, np.complex128, (0.25, -0.125, 0.375)),
+    ((40, 48, 46), True, 40, np.complex64, (0.25, 0.1, 0.3))])
+def test_unsymmetric_coefficients(monkeypatch, N_c, pbc, nb, dtype, k_c,
+                                  kernel):
+    """Different coefficients at +j and -j (a one-sided derivative)."""
+    monkeypatch.setenv('GPAW_AMD_STENCIL', kernel)
+    rng = np.random.default_rng(8)
+    N_c = np.array(N_c)
+    gd = GridDescriptor(N_c, N_c * 0.4, pbc)
+    ogd = og.Grid(N_c, N_c * 0.4, pbc)
+    offs = [(0, 0, 0)] + [tuple(s * j if c == d else 0 for d in range(3))
+                          for c in range(3) for j in (1, 2) for s in (1, -1)]
+    coef = rng.uniform(-1, 1, len(offs))
+    cplx = np.dtype(dtype).kind == 'c'
+    shape = (nb,) + tuple(gd.n_c)
+    a = rng.standard_normal(shape)
+    a = (a + 1j * rng.standard_normal(shape) if cplx else a).astype(dtype)
+    ph = None if k_c is None else ogd.phase_cd(k_c)
+    pick = sorted({0, nb // 2, nb - 1})
+    ref = ost.fd_apply(coef, np.array(offs), a[pick].astype(
+        np.complex128 if cplx else np.float64), ogd.pbc_c, ph)
+    op = FDOperator(coef, offs, gd, dtype)
+    d = torch.from_numpy(a).cuda()
+    out = torch.empty_like(d)
+    op.apply(d, out, ph)
+    tol = 2e-5 if dtype in (np.float32, np.complex64) else 1e-12
+    assert abs(out[pick].cpu().numpy() - ref).max() < tol * abs(ref).max()
