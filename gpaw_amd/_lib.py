@@ -13,6 +13,7 @@ LIB_PATH = os.path.join(HERE, 'lib', 'libgpawhip.so')
 
 GH_F64, GH_C128, GH_F32, GH_C64 = 0, 1, 2, 3
 GH_DOT_CHUNKS = 64
+GH_ERR_UNSUPPORTED = -4
 
 _c = ctypes
 P = _c.c_void_p
@@ -78,6 +79,10 @@ _SIGNATURES = {
     'gh_unet_conv3': (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int,
                                  _c.c_int, PI64, P, P, P, P, P, D, P, P,
                                  _c.c_int, P, P]),
+    'gh_unet_conv3_map1': (_c.c_int, [_c.c_int, PI64, P, P, P, P, P, P, P,
+                                      P]),
+    'gh_unet_conv3_head': (_c.c_int, [_c.c_int, _c.c_int, PI64, P, P, P, P, P,
+                                      D, P, P, P]),
     'gh_unet_pool2': (_c.c_int, [_c.c_int, _c.c_int, PI64, P, P, P]),
     'gh_unet_map1': (_c.c_int, [_c.c_int, _c.c_int, I64, P, P, P, P, P]),
     'gh_unet_head': (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, I64, P, P, D,

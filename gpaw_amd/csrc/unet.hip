@@ -26,8 +26,10 @@
 // memory-bound element kernels.
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
+#include "internal.h"
 
 namespace gh {
 
@@ -46,6 +48,18 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
     u += 0x7fffu + ((u >> 16) & 1u);
     return (unsigned short)(u >> 16);
 }
+
+// two values, round to nearest even, in one instruction (low half: a)
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned f2bf2(float a, float b) {
+    const b2v r = __builtin_convertvector((f2v{a, b}), b2v);
+    unsigned u;
+    __builtin_memcpy(&u, &r, 4);
+    return u;
+}
+__device__ __forceinline__ float bf_lo(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf_hi(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
 
 enum { kFirst = 0, kPlain = 1, kUpAdd = 2 };
 
@@ -274,6 +288,318 @@ conv3_lds_kernel(ConvGeom g, int ty, const unsigned short* __restrict__ in,
     }
 }
 
+// The convolution of the two fine levels (C_in <= 16, C_out <= 16), marching
+// along x.  A block owns one band, ty full rows and lx planes; a ring of
+// four planes (its rows and halo, periodic images included) is in LDS, every
+// plane is loaded into registers one iteration ahead and staged once (the
+// per-plane kernel above stages three planes for every plane it computes),
+// and there is one barrier per plane.
+//   * The products are formed as W^T A^T: a lane ends with four channels of
+//     one point, so results leave in 8-byte stores, and what follows the
+//     layer can work on them in registers: kHead, the final 1x1 map to the
+//     correction, and kMap, the 1x1 map 16 -> 8 that precedes the upsampling.
+//   * The taps' LDS offsets are uniform, so a product costs a selection and
+//     an add, one 8-byte LDS read and the matrix instruction.  Two 16-point
+//     tiles per wave interleave their chains.
+// The order of the products and sums of a result is that of the kernel above
+// (same k-chunks, same instruction), so are its bits.
+// Bounds: staging and epilogue instructions and LDS reads; activations move
+// 16 to 40 bytes per point.  64 bands of 96^3 (48^3 on the coarse level), us,
+// the per-plane kernel and the map's own pass -> here:
+//   2 -> 8 first layer             2609        -> 519  (bytes: 270)
+//   8 -> 16 coarse                  435        -> 118
+//   16 -> 16 upsampled + 16 -> 8    905 + 203  -> 382
+//   8 -> 8 upsampled + correction  4528 + 220  -> 860  (bytes: 290)
+enum { kStore = 0, kHead = 1, kMap = 2 };
+
+template <typename T>
+struct MarchOut {
+    unsigned short* act;      // kStore: channel-last result; kMap: 8 channels
+    T* corr;                  // kHead: the correction
+    const float* W;           // kHead: W[c]; kMap: W[ci][8]
+    const float* bias;        // kMap: 8 values
+    const float* scale;       // kHead: per band
+    float bias0;              // kHead
+};
+
+constexpr int kMarchThreads = 512;
+// staged items per thread and plane (each up to 8 registers)
+template <int CL> struct MarchItems { static constexpr int value = CL == 4 ? 4 : 2; };
+
+template <int CIN, int COUT, int MODE, int EPI, typename T>
+__global__ void __launch_bounds__(kMarchThreads, CIN == 16 ? 2 : 4)
+conv3_march_kernel(ConvGeom g, int ty, int lx, int nyt, int nxc, unsigned zmagic,
+                   const unsigned short* __restrict__ in,
+                   const unsigned short* __restrict__ skip, FirstIn<T> fin,
+                   const unsigned short* __restrict__ W, const float* __restrict__ bias,
+                   int relu, MarchOut<T> o) {
+    constexpr int CL = MODE == kFirst ? 4 : CIN;
+    // Staged points are PB bytes apart; 16 channels are two halves of 8 in
+    // planes of their own (32 bytes apart, the 16 points of a read would meet
+    // in the same LDS banks twice).
+    constexpr int PB = CL >= 8 ? 16 : 8;
+    constexpr int IPP = 2 * CL / PB;                  // items of PB bytes per point
+    constexpr int NK = (27 * CL + 15) / 16;
+    constexpr int NI = MarchItems<CL>::value;
+    static_assert(COUT <= 16 && CL <= 16, "one column tile");
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = lane >> 4, row = lane & 15;
+    int L = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int yt = L % nyt;
+    L /= nyt;
+    const int xc = L % nxc, b = L / nxc;
+    const int y0 = yt * ty, tye = min(ty, g.ny - y0);
+    const int x0 = xc * lx, x1 = min(x0 + lx, g.nx);
+    const int nz = g.nz, nzp = nz + 2;
+    const int half = (ty + 2) * nzp * PB, slab = half * IPP;
+    const int64_t plane = (int64_t)g.ny * nz;
+    const int cny = g.ny / 2, cnz = g.nz / 2;
+    const int64_t cplane = (int64_t)cny * cnz;
+    const int nitem = (tye + 2) * nzp * IPP;
+    const int npts = tye * nz;
+
+    // staged items of this thread: offset in the plane (and coarse plane),
+    // in elements
+    int goff[NI], coff[NI];
+#pragma unroll
+    for (int u = 0; u < NI; u++) {
+        const int it = min(tid + u * kMarchThreads, nitem - 1);
+        const int q = it / IPP, c = (it - q * IPP) * (PB / 2);
+        const int yl = q / nzp, zl = q - yl * nzp;
+        int yy = y0 + yl - 1, zz = zl - 1;
+        yy += yy < 0 ? g.ny : (yy >= g.ny ? -g.ny : 0);
+        zz += zz < 0 ? nz : (zz >= nz ? -nz : 0);
+        goff[u] = MODE == kFirst ? yy * nz + zz : (yy * nz + zz) * CIN + c;
+        coff[u] = MODE == kUpAdd ? ((yy >> 1) * cnz + (zz >> 1)) * CIN + c : 0;
+    }
+    struct Raw { u4 a, c; T r, v; };
+    Raw raw[NI];
+    const float sc = MODE == kFirst ? fin.scale[b] : 0.f;
+    auto load = [&](int xp) {
+        const int xx = xp < 0 ? xp + g.nx : (xp >= g.nx ? xp - g.nx : xp);
+        if constexpr (MODE == kFirst) {
+            const T* R = fin.R + ((int64_t)b * g.nx + xx) * plane;
+            const T* v = fin.v + xx * plane;
+#pragma unroll
+            for (int u = 0; u < NI; u++)
+                if (tid + u * kMarchThreads < nitem) {
+                    raw[u].r = R[goff[u]];
+                    raw[u].v = v[goff[u]];
+                }
+        } else {
+            const unsigned short* f =
+                (MODE == kPlain ? in : skip) + ((int64_t)b * g.nx + xx) * plane * CIN;
+            const unsigned short* c =
+                MODE == kUpAdd ? in + ((int64_t)b * (g.nx / 2) + (xx >> 1)) * cplane * CIN : in;
+#pragma unroll
+            for (int u = 0; u < NI; u++)
+                if (tid + u * kMarchThreads < nitem) {
+                    raw[u].a = *reinterpret_cast<const u4*>(f + goff[u]);
+                    if (MODE == kUpAdd) raw[u].c = *reinterpret_cast<const u4*>(c + coff[u]);
+                }
+        }
+    };
+    auto stage = [&](int slot) {
+        unsigned char* ring = smem_raw + slot * slab;
+#pragma unroll
+        for (int u = 0; u < NI; u++) {
+            const int it = tid + u * kMarchThreads;
+            if (it >= nitem) continue;
+            unsigned char* d = ring + (it % IPP) * half + (it / IPP) * PB;
+            if constexpr (MODE == kFirst) {
+                const float r = (float)raw[u].r * sc, v = (float)raw[u].v * fin.vscale;
+                *reinterpret_cast<u2*>(d) = u2{f2bf2(r, v), 0u};
+            } else if constexpr (MODE == kPlain) {
+                *reinterpret_cast<u4*>(d) = raw[u].a;
+            } else {
+                u4 s;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const unsigned p = raw[u].a[e], q = raw[u].c[e];
+                    s[e] = f2bf2(bf_lo(p) + bf_lo(q), bf_hi(p) + bf_hi(q));
+                }
+                *reinterpret_cast<u4*>(d) = s;
+            }
+        }
+    };
+
+    // A k-chunk of 16 covers 16 / CL taps; this lane's is tap
+    // kc 16 / CL + 4 grp / CL, its channels 4 grp % CL ...  The taps' offsets
+    // in the ring are uniform (sb: slots of the planes x - 1, x, x + 1), so
+    // only the selection between a chunk's taps is the lane's own.  A tap
+    // beyond the last reads tap 26 and counts as zero.
+    constexpr int TPC = 16 / CL;
+    int sb[3] = {0, 0, 0};
+    const int own = IPP == 2 ? (grp >> 1) * half + 8 * (grp & 1) : 2 * (4 * grp % CL);
+    const int sub = 4 * grp / CL;
+    auto tap_off = [&](int tap) {
+        tap = tap < 27 ? tap : 26;
+        return sb[tap / 9] + (((tap / 3) % 3) * nzp + tap % 3) * PB;
+    };
+    auto chunk_off = [&](int kc) {
+        int v = tap_off(kc * TPC);
+#pragma unroll
+        for (int t = 1; t < TPC; t++) v = sub == t ? tap_off(kc * TPC + t) : v;
+        return v;
+    };
+    const bool tail = 16 * (NK - 1) + 4 * grp >= 27 * CL;
+    bf4 wr[NK];
+#pragma unroll
+    for (int kc = 0; kc < NK; kc++)
+        wr[kc] = *reinterpret_cast<const bf4*>(W + ((int64_t)kc * 64 + lane) * 4);
+    float bv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) bv[r] = 4 * grp + r < COUT ? bias[4 * grp + r] : 0.f;
+    float mw[EPI == kMap ? 32 : 1];       // kMap: the weights of this lane's two results
+    if constexpr (EPI == kMap) {
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            mw[2 * c] = o.W[c * 8 + 2 * grp];
+            mw[2 * c + 1] = o.W[c * 8 + 2 * grp + 1];
+        }
+    }
+    float hw[4];
+    float inv_scale = 1.f;
+    if constexpr (EPI == kHead) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) hw[r] = o.W[(4 * grp + r) & 7];
+        inv_scale = o.scale[b];
+    }
+
+    // one result tile: channels 4 grp .. of point p
+    unsigned short* oact = nullptr;      // this lane's channels of the plane's first point
+    T* ocorr = nullptr;
+    const float mb0 = EPI == kMap ? o.bias[2 * grp] : 0.f;
+    const float mb1 = EPI == kMap ? o.bias[2 * grp + 1] : 0.f;
+    auto finish = [&](f4v acc, int p) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            v[r] = acc[r] + bv[r];
+            if (relu) v[r] = fmaxf(v[r], 0.f);
+        }
+        const u2 h = u2{f2bf2(v[0], v[1]), f2bf2(v[2], v[3])};
+        if constexpr (EPI == kStore) {
+            if (p < npts && 4 * grp < COUT) *reinterpret_cast<u2*>(oact + p * COUT) = h;
+        } else if constexpr (EPI == kHead) {
+            // the sum over channels in order: lane group 0, then group 1
+            const float f[4] = {bf_lo(h.x), bf_hi(h.x), bf_lo(h.y), bf_hi(h.y)};
+            float s = o.bias0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) s += hw[r] * f[r];
+            s = __shfl(s, row);
+#pragma unroll
+            for (int r = 0; r < 4; r++) s += hw[r] * f[r];
+            if (grp == 1 && p < npts) ocorr[p] = (T)(s / inv_scale);
+        } else {
+            // every lane gathers the point's 16 channels and forms two of
+            // the 8 results
+            float s0 = mb0, s1 = mb1;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const unsigned p0 = (unsigned)__shfl((int)h.x, 16 * q + row);
+                const unsigned p1 = (unsigned)__shfl((int)h.y, 16 * q + row);
+                const float f[4] = {bf_lo(p0), bf_hi(p0), bf_lo(p1), bf_hi(p1)};
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    s0 += mw[2 * (4 * q + r)] * f[r];
+                    s1 += mw[2 * (4 * q + r) + 1] * f[r];
+                }
+            }
+            if (p < npts) *reinterpret_cast<unsigned*>(oact + p * 8) = f2bf2(s0, s1);
+        }
+    };
+
+    // slot of plane xp: (xp - x0 + 1) mod 4
+    load(x0 - 1);
+    stage(0);
+    load(x0);
+    stage(1);
+    load(x0 + 1);
+    stage(2);
+    __syncthreads();
+    constexpr int NW = kMarchThreads / 64;
+    for (int x = x0; x < x1; x++) {
+        const bool more = x + 1 < x1;
+        if (more) load(x + 2);                 // in flight during this plane
+#pragma unroll
+        for (int d = 0; d < 3; d++) sb[d] = ((x - x0 + d) & 3) * slab;
+        const int64_t pt0 = ((int64_t)b * g.nx + x) * plane + (int64_t)y0 * nz;
+        if constexpr (EPI == kHead) ocorr = o.corr + pt0;
+        else oact = o.act + pt0 * (EPI == kMap ? 8 : COUT) + (EPI == kMap ? 2 : 4) * grp;
+        for (int p0 = wave * 16; p0 < npts; p0 += 2 * NW * 16) {
+            const int pa = p0 + row, pb = pa + NW * 16;
+            const unsigned ca = min(pa, npts - 1), cb = min(pb, npts - 1);
+            const int ya = (int)__umulhi(ca, zmagic), yb = (int)__umulhi(cb, zmagic);
+            // ca / nz by the magic factor; slab offset of the point
+            const int ba = (ya * nzp + (int)ca - ya * nz) * PB + own;
+            const int bb = (yb * nzp + (int)cb - yb * nz) * PB + own;
+            f4v acca = f4v{0.f, 0.f, 0.f, 0.f}, accb = acca;
+            const bool two = p0 + NW * 16 < npts;      // wave-uniform
+            auto chain = [&](auto both) {
+#pragma unroll
+                for (int kc = 0; kc < NK; kc++) {
+                    const int off = chunk_off(kc);
+                    const bool zero = kc == NK - 1 && (27 * CL) % 16 != 0 && tail;
+                    bf4 a = *reinterpret_cast<const bf4*>(smem_raw + ba + off);
+                    if (zero) a = bf4{0, 0, 0, 0};
+                    acca = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wr[kc], a, acca, 0, 0, 0);
+                    if constexpr (decltype(both)::value) {
+                        bf4 c = *reinterpret_cast<const bf4*>(smem_raw + bb + off);
+                        if (zero) c = bf4{0, 0, 0, 0};
+                        accb = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wr[kc], c, accb, 0, 0, 0);
+                    }
+                }
+            };
+            if (two) chain(std::true_type{});
+            else chain(std::false_type{});
+            finish(acca, pa);
+            if (two) finish(accb, pb);
+        }
+        if (more) stage((x - x0 + 3) & 3);
+        __syncthreads();
+    }
+}
+
+// Launch of the marching form; GH_ERR_UNSUPPORTED when a row does not fit.
+template <int CIN, int COUT, int MODE, int EPI, typename T>
+int launch_march(const ConvGeom& g, const void* in, const void* skip, const FirstIn<T>& fin,
+                 const void* W, const float* bias, int relu, const MarchOut<T>& o,
+                 hipStream_t st) {
+    constexpr int CL = MODE == kFirst ? 4 : CIN;
+    constexpr int PB = 2 * CL, IPP = PB < 16 ? 1 : PB / 16;
+    const int nzp = g.nz + 2;
+    // rows: 80 KB of LDS (two blocks per CU) and MarchItems items per thread
+    const int64_t lds_row = 4LL * nzp * PB;
+    int ty = (int)std::min<int64_t>(g.ny, std::min<int64_t>(80 * 1024 / lds_row,
+                                        (int64_t)MarchItems<CL>::value * kMarchThreads / (nzp * IPP)) - 2);
+    if (ty < 1 || g.nz < 2 || (int64_t)g.ny * g.nz * CIN >= (1ll << 31)) return GH_ERR_UNSUPPORTED;
+    const int nyt = (g.ny + ty - 1) / ty;
+    ty = (g.ny + nyt - 1) / nyt;
+    // x-runs: two blocks per CU four times over where the grid allows it
+    // (each run stages two planes more), at least 8 planes
+    const int64_t base = (int64_t)g.nbands * nyt;
+    int nxc = (int)std::min<int64_t>(std::max(1, g.nx / 8), std::max<int64_t>(1, 2048 / base));
+    const int lx = (g.nx + nxc - 1) / nxc;
+    nxc = (g.nx + lx - 1) / lx;
+    const int64_t nblk = base * nxc;
+    GH_REQUIRE(nblk < (1ll << 31), GH_ERR_SHAPE, "unet_conv3: too many blocks");
+    const size_t lds = (size_t)lds_row * (ty + 2);
+    auto kfn = conv3_march_kernel<CIN, COUT, MODE, EPI, T>;
+    const int rc = ensure_max_lds((const void*)kfn, 160 * 1024);
+    if (rc != GH_OK) return rc;
+    const unsigned magic = (unsigned)(((1ull << 32) + g.nz - 1) / g.nz);
+    hipLaunchKernelGGL(kfn, dim3((unsigned)nblk), dim3(kMarchThreads), lds, st, g, ty, lx, nyt,
+                       nxc, magic, (const unsigned short*)in, (const unsigned short*)skip, fin,
+                       (const unsigned short*)W, bias, relu, o);
+    GH_CHECK_LAUNCH();
+    return GH_OK;
+}
+
 // 2x2x2 average of a channel-last BF16 tensor (fine grid nx, ny, nz even).
 template <int C>
 __global__ void __launch_bounds__(256)
@@ -332,6 +658,13 @@ template <int CIN, int COUT, int MODE, typename T>
 int launch_conv3(const ConvGeom& g, const void* in, const void* skip, const FirstIn<T>& fin,
                  const void* W, const float* bias, int relu, void* out, hipStream_t st) {
     constexpr int CL = MODE == kFirst ? 4 : CIN;
+    if constexpr (CIN <= 16 && COUT <= 16) {
+        MarchOut<T> o{};
+        o.act = (unsigned short*)out;
+        const int rc = launch_march<CIN, COUT, MODE, kStore, T>(g, in, skip, fin, W, bias, relu,
+                                                                o, st);
+        if (rc != GH_ERR_UNSUPPORTED) return rc;
+    }
     const int64_t per_row = 3LL * (g.nz + 2) * CL * 2;
     const int ty = (int)std::min<int64_t>(g.ny, kConvLds / per_row - 2);
     if (ty >= 1) {
@@ -445,6 +778,62 @@ int gh_unet_conv3(int cin, int cout, int mode, int dtype, int nbands, const int6
 #undef GH_CONV
     set_error("unet_conv3: layer %d -> %d (mode %d) not built", cin, cout, mode);
     return GH_ERR_UNSUPPORTED;
+}
+
+int gh_unet_conv3_map1(int nbands, const int64_t* n_c, const void* in_dev, const void* skip_dev,
+                       const void* W_dev, const float* bias_dev, const float* Wm_dev,
+                       const float* bm_dev, void* out_dev, void* stream) {
+    GH_REQUIRE(n_c && W_dev && bias_dev && Wm_dev && bm_dev && nbands >= 0, GH_ERR_ARG,
+               "unet_conv3_map1: null argument");
+    if (nbands == 0) return GH_OK;
+    ConvGeom g{(int)n_c[0], (int)n_c[1], (int)n_c[2], nbands};
+    GH_REQUIRE(g.nx >= 2 && g.ny >= 2 && g.nz >= 2 && g.nx % 2 == 0 && g.ny % 2 == 0 &&
+                   g.nz % 2 == 0 && in_dev && skip_dev && out_dev,
+               GH_ERR_SHAPE, "unet_conv3_map1: upsampling needs an even grid and a skip");
+    MarchOut<float> o{};
+    o.act = (unsigned short*)out_dev;
+    o.W = Wm_dev;
+    o.bias = bm_dev;
+    const int rc = launch_march<16, 16, kUpAdd, kMap, float>(
+        g, in_dev, skip_dev, FirstIn<float>{}, W_dev, bias_dev, 1, o, (hipStream_t)stream);
+    if (rc == GH_ERR_UNSUPPORTED) set_error("unet_conv3_map1: rows of %d points", g.nz);
+    return rc;
+}
+
+int gh_unet_conv3_head(int dtype, int nbands, const int64_t* n_c, const void* in_dev,
+                       const void* skip_dev, const void* W_dev, const float* bias_dev,
+                       const float* Wh_dev, double bias, const float* scale_dev, void* out_dev,
+                       void* stream) {
+    GH_REQUIRE(n_c && W_dev && bias_dev && Wh_dev && nbands >= 0, GH_ERR_ARG,
+               "unet_conv3_head: null argument");
+    GH_REQUIRE(dtype == GH_F32 || dtype == GH_F64, GH_ERR_UNSUPPORTED,
+               "unet_conv3_head: real outputs only");
+    if (nbands == 0) return GH_OK;
+    ConvGeom g{(int)n_c[0], (int)n_c[1], (int)n_c[2], nbands};
+    GH_REQUIRE(g.nx >= 2 && g.ny >= 2 && g.nz >= 2 && g.nx % 2 == 0 && g.ny % 2 == 0 &&
+                   g.nz % 2 == 0 && in_dev && skip_dev && out_dev && scale_dev,
+               GH_ERR_SHAPE, "unet_conv3_head: upsampling needs an even grid and a skip");
+    int rc;
+    if (dtype == GH_F32) {
+        MarchOut<float> o{};
+        o.corr = (float*)out_dev;
+        o.W = Wh_dev;
+        o.scale = scale_dev;
+        o.bias0 = (float)bias;
+        rc = launch_march<8, 8, kUpAdd, kHead, float>(g, in_dev, skip_dev, FirstIn<float>{},
+                                                      W_dev, bias_dev, 1, o, (hipStream_t)stream);
+    } else {
+        MarchOut<double> o{};
+        o.corr = (double*)out_dev;
+        o.W = Wh_dev;
+        o.scale = scale_dev;
+        o.bias0 = (float)bias;
+        rc = launch_march<8, 8, kUpAdd, kHead, double>(g, in_dev, skip_dev, FirstIn<double>{},
+                                                       W_dev, bias_dev, 1, o,
+                                                       (hipStream_t)stream);
+    }
+    if (rc == GH_ERR_UNSUPPORTED) set_error("unet_conv3_head: rows of %d points", g.nz);
+    return rc;
 }
 
 int gh_unet_pool2(int c, int nbands, const int64_t* n_c, const void* in_dev, void* out_dev,

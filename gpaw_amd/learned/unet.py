@@ -185,15 +185,36 @@ class HIPUNet:
         self._conv('c2b', 32, 32, 1, nb, n2, e2, inp=t2)
         u2 = self._act('u2', (p2, 16))
         self._map('m2', 32, 16, p2, e2, u2)
-        h1 = self._act('h1', (p1, 16))
-        self._conv('c1u', 16, 16, 2, nb, n1, h1, inp=u2, skip=e1)
+        # c1u and its map, c0u and the head: one pass each where the rows
+        # fit the kernel, else layer by layer
         u1 = self._act('u1', (p1, 8))
-        self._map('m1', 16, 8, p1, h1, u1)
-        h0 = self._act('h0', (p0, 8))
-        self._conv('c0u', 8, 8, 2, nb, n0, h0, inp=u1, skip=e0)
+        W, b = self.conv['c1u']
+        Wm, bm = self.map1['m1']
+        n = np.ascontiguousarray(n1, np.int64)
+        rc = self._lib.gh_unet_conv3_map1(
+            nb, n.ctypes.data_as(_lib.PI64), u2.data_ptr(), e1.data_ptr(),
+            W.data_ptr(), b.data_ptr(), Wm.data_ptr(), bm.data_ptr(),
+            u1.data_ptr(), stream_ptr())
+        if rc == _lib.GH_ERR_UNSUPPORTED:
+            h1 = self._act('h1', (p1, 16))
+            self._conv('c1u', 16, 16, 2, nb, n1, h1, inp=u2, skip=e1)
+            self._map('m1', 16, 8, p1, h1, u1)
+        else:
+            _lib.check(rc)
+        W, b = self.conv['c0u']
         Wh, bh = self.map1['head']
-        _lib.check(self._lib.gh_unet_head(
-            8, dtype_code(out.dtype), nb, p0 // nb, h0.data_ptr(),
+        n = np.ascontiguousarray(n0, np.int64)
+        rc = self._lib.gh_unet_conv3_head(
+            dtype_code(out.dtype), nb, n.ctypes.data_as(_lib.PI64),
+            u1.data_ptr(), e0.data_ptr(), W.data_ptr(), b.data_ptr(),
             Wh.data_ptr(), self.head_bias, scale.data_ptr(), out.data_ptr(),
-            stream_ptr()))
+            stream_ptr())
+        if rc == _lib.GH_ERR_UNSUPPORTED:
+            h0 = self._act('h0', (p0, 8))
+            self._conv('c0u', 8, 8, 2, nb, n0, h0, inp=u1, skip=e0)
+            rc = self._lib.gh_unet_head(
+                8, dtype_code(out.dtype), nb, p0 // nb, h0.data_ptr(),
+                Wh.data_ptr(), self.head_bias, scale.data_ptr(),
+                out.data_ptr(), stream_ptr())
+        _lib.check(rc)
         return out

@@ -378,6 +378,20 @@ int gh_unet_conv3(int cin, int cout, int mode, int dtype, int nbands,
                   const void* R_dev, const void* v_dev, const float* scale_dev,
                   double vscale, const void* W_dev, const float* bias_dev,
                   int relu, void* out_dev, void* stream);
+/* A mode-2 layer (with relu) and the 1x1 map that follows it, in one pass
+ * (the layer's own result is not stored): 16 -> 16 then the map
+ * Wm[ci][8] / bm to 8 channels; 8 -> 8 then the correction of gh_unet_head.
+ * The same bits as the two calls.  GH_ERR_UNSUPPORTED for rows too long for
+ * the LDS: use the two calls. */
+int gh_unet_conv3_map1(int nbands, const int64_t* n_c, const void* in_dev,
+                       const void* skip_dev, const void* W_dev,
+                       const float* bias_dev, const float* Wm_dev,
+                       const float* bm_dev, void* out_dev, void* stream);
+int gh_unet_conv3_head(int dtype, int nbands, const int64_t* n_c,
+                       const void* in_dev, const void* skip_dev,
+                       const void* W_dev, const float* bias_dev,
+                       const float* Wh_dev, double bias,
+                       const float* scale_dev, void* out_dev, void* stream);
 /* 2x2x2 average pooling (fine grid n_c, even), c = 8, 16 or 32. */
 int gh_unet_pool2(int c, int nbands, const int64_t* n_c, const void* in_dev,
                   void* out_dev, void* stream);
