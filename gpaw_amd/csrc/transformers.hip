@@ -19,6 +19,7 @@
 // registers), and keeps the last 2K-1 (restrict) or K (interpolate) filtered
 // planes in a register queue that the x-filter reads.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
@@ -612,33 +613,60 @@ constexpr int ppt_of(bool interp) {
     return (!interp && (K >= 6 || sizeof(V) > 8)) ? 1 : 2;
 }
 
-// Rows of the output tile: as many as fit 1024 threads and 64 KB LDS.
-int choose_rows(const gh_transformer* h, int vsize, int ppt, size_t* lds_out,
-                int* nry_out) {
+// Tile (output rows) and x-run of a block: the pair with the least estimated
+// time.  A block walks its run's input planes (the first ones only prime the
+// filter queue); a plane costs two barriers and their latency, about the time
+// of 6 KB at a CU's share of the HBM rate, plus what every block beside it on
+// the CU moves through HBM and, at a fifteenth, through LDS.  Blocks beyond
+// what the CUs hold go into further rounds.  Cutting the runs until 2048
+// blocks existed, as before, primed 9 to 11 planes for every 8: 2 densities
+// 112^3 -> 224^3 with nn = 3 took 119 us and take 60, 128 complex64 functions
+// restricted from 112^3 with nn = 3 684 and 520 us, 16 FP32 functions 48^3 with
+// nn = 1 14.6 and 8.2 us.
+struct TTile {
+    int tj = 0, lx = 0, nry = 0;
+    size_t lds = 0;
+};
+
+TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, int ncu) {
     const TGeom& g = h->g;
     const int K = 2 * h->nn;
-    int best = 0;
-    size_t best_lds = 0;
-    int best_nry = 0;
-    // the 2-tap restriction (V-cycle) is fastest with short tiles and more
-    // blocks (measured at 112^3 -> 56^3, 256 bands: 4-17 % over 14 rows)
-    const int maxrows = (!h->interp && h->nn == 1) ? 7 : g.m[1];
-    for (int tj = 1; tj <= std::min(g.m[1], maxrows); tj++) {
-        int nry = h->interp ? (tj + 1) / 2 + 2 * h->nn + 1 : 2 * tj + 2 * K - 3;
+    TTile best;
+    double tbest = 0;
+    for (int tj = 1; tj <= g.m[1]; tj++) {
+        const int nry = h->interp ? (tj + 1) / 2 + 2 * h->nn + 1 : 2 * tj + 2 * K - 3;
         // interpolation: staged rows + their z-filtered rows; restriction:
         // staged rows + the tile's y-filtered rows (full staged width)
-        size_t lds = h->interp ? (size_t)nry * (g.zw + g.m[2]) * vsize
-                               : (size_t)(nry + tj) * g.zw * vsize;
-        int thr = (tj * g.m[2] + ppt - 1) / ppt;
+        const size_t lds = h->interp ? (size_t)nry * (g.zw + g.m[2]) * vsize
+                                     : (size_t)(nry + tj) * g.zw * vsize;
+        const int thr = ((tj * g.m[2] + ppt - 1) / ppt + 63) / 64 * 64;
         if (lds > 64 * 1024 || thr > 1024) break;
-        if (g.m[1] % tj == 0 || tj == g.m[1] || best == 0) {
-            best = tj;
-            best_lds = lds;
-            best_nry = nry;
+        const int64_t nyt = (g.m[1] + tj - 1) / tj;
+        const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(2048 / thr, 160 * 1024 / lds));
+        const double hbm = ((double)nry * g.zw +
+                            (h->interp ? 2.0 : 0.5) * tj * g.m[2]) * vsize;
+        const double taps = h->interp ? (K + 2) / 2.0 * (nry * g.m[2] + tj * g.m[2])
+                                      : (K + 2.0) * (tj * g.zw + tj * g.m[2]);
+        const double plane = hbm + taps * vsize / 15;
+        const double room = (double)ncu * fit;
+        // steps of an eighth: a few microseconds per call for this search
+        for (int nxc = 1; nxc <= std::max(1, g.m[0] / 2); nxc += 1 + nxc / 8) {
+            const int lx = (g.m[0] + nxc - 1) / nxc;
+            const double blocks = (double)(nbands * nyt) * ((g.m[0] + lx - 1) / lx);
+            const double rounds = std::ceil(blocks / room);
+            const double beside = std::min((double)fit, std::ceil(blocks / ncu));
+            const double planes = h->interp ? (lx + 1) / 2 + K - 1 : 2 * lx + 2 * K - 3;
+            const double t = rounds * planes * (beside * plane + 6144.0);
+            if (best.tj == 0 || t < tbest) {
+                tbest = t;
+                best.tj = tj;
+                best.lx = lx;
+                best.nry = nry;
+                best.lds = lds;
+            }
+            if (rounds > 4) break;
         }
     }
-    *lds_out = best_lds;
-    *nry_out = best_nry;
     return best;
 }
 
@@ -647,24 +675,22 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
              int64_t nbands, const double* phase_cd, double alpha,
              hipStream_t st) {
     TGeom g = h->g;
-    size_t lds;
-    int nry;
     constexpr int PPT_R = ppt_of<V, K>(false);
     constexpr int PPT_I = ppt_of<V, K>(true);
     const int ppt = h->interp ? PPT_I : PPT_R;
-    int tj = choose_rows(h, sizeof(V), ppt, &lds, &nry);
-    GH_REQUIRE(tj > 0, GH_ERR_UNSUPPORTED,
+    int ncu = 0;
+    const int crc = device_cu_count(&ncu);
+    if (crc != GH_OK) return crc;
+    const TTile tile = choose_tile(h, sizeof(V), ppt, nbands, ncu);
+    GH_REQUIRE(tile.tj > 0, GH_ERR_UNSUPPORTED,
                "transformer: grid rows too long for one block");
+    const int tj = tile.tj;
+    const size_t lds = tile.lds;
     g.tj = tj;
-    g.nry = nry;
-    g.lx = g.m[0];
+    g.nry = tile.nry;
+    g.lx = tile.lx;
     g.nyt = (g.m[1] + tj - 1) / tj;
-    g.nxc = 1;
-    // split x so that there are enough blocks to fill the GPU
-    while ((int64_t)nbands * g.nyt * g.nxc < 2048 && g.lx > 8) {
-        g.lx = (g.lx + 1) / 2;
-        g.nxc = (g.m[0] + g.lx - 1) / g.lx;
-    }
+    g.nxc = (g.m[0] + g.lx - 1) / g.lx;
     int thr = (tj * g.m[2] + ppt - 1) / ppt;
     thr = ((thr + 63) / 64) * 64;
     int64_t nblocks = nbands * (int64_t)g.nyt * g.nxc;
