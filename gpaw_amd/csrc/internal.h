@@ -40,6 +40,23 @@ int stencil_rows(int dtype, const DirectStencil& h, const void* in, void* out,
                  const void* src, double beta, double alpha, double gamma,
                  const double* eps, int ncu, hipStream_t st);
 
+// The stencil as axis coefficients; false for another form, or where
+// GPAW_AMD_STENCIL names a kernel
+bool stencil_axes(const gh_stencil* h, DirectStencil* out);
+
+// Linear interpolation to the grid of half the spacing
+struct InterpGrid {
+    int n[3], plo[3], skip[3], pbc[3];   // coarse grid, ghosts below, points skipped
+};
+bool transformer_interp(const gh_transformer* h, int dtype, InterpGrid* out);
+
+// out = al * (L I u) + ga * I u + sum_q beta[q] src[q] (1 or 2 sources), I the
+// interpolation (stencil_interp.hip); GH_ERR_UNSUPPORTED where that kernel
+// has no path
+int stencil_interp(const gh_stencil* h, const gh_transformer* intp, const void* u, void* out,
+                   int64_t nb, const double* phase_cd, int ns, const void* const* src,
+                   const double* beta, double al, double ga, hipStream_t st);
+
 int device_cu_count(int* out);
 int ensure_max_lds(const void* kernel, int bytes);
 

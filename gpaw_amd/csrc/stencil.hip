@@ -732,10 +732,7 @@ constexpr size_t kLdsBytes = 160 * 1024;
 template <typename V> struct RingPPT { static constexpr int value = 2; };
 template <> struct RingPPT<float> { static constexpr int value = 4; };
 
-template <typename V, typename S>
-int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
-               const double* ph, const void* vt, const void* src, double beta,
-               double al, double ga, const double* eps, hipStream_t st) {
+DirectStencil axes_of(const gh_stencil* h) {
     DirectStencil d;
     for (int c = 0; c < 3; c++) {
         d.n[c] = (int)h->n[c];
@@ -749,6 +746,14 @@ int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
     d.c0 = h->c0;
     d.rows = h->ty_req;
     d.planes = h->lx_req;
+    return d;
+}
+
+template <typename V, typename S>
+int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
+               const double* ph, const void* vt, const void* src, double beta,
+               double al, double ga, const double* eps, hipStream_t st) {
+    const DirectStencil d = axes_of(h);
     // The LDS ring needs a few MB to fill the GPU with its large blocks; up to
     // 5 MB the kernel without LDS, split as finely as it likes, is faster:
     // FP64, R = 3, 2 x 64^3 (4.2 MB) 7.3 against 8.6 us, 96^3 (7.1 MB) 9.8
@@ -1236,6 +1241,12 @@ namespace gh {
 
 int64_t stencil_points(const gh_stencil* h) { return h->n[0] * h->n[1] * h->n[2]; }
 int stencil_dtype(const gh_stencil* h) { return h->dtype; }
+
+bool stencil_axes(const gh_stencil* h, DirectStencil* out) {
+    if (!h->cfd || h->mode != 0) return false;
+    *out = axes_of(h);
+    return true;
+}
 
 int stencil_apply_scaled(const gh_stencil* h, const void* in_dev, void* out_dev,
                          int64_t nbands, const double* phase_cd,

@@ -826,6 +826,17 @@ int64_t transformer_out_points(const gh_transformer* h) {
     return (int64_t)h->g.m[0] * h->g.m[1] * h->g.m[2];
 }
 
+bool transformer_interp(const gh_transformer* h, int dtype, InterpGrid* out) {
+    if (!h->interp || h->nn != 1 || h->dtype != dtype) return false;
+    for (int c = 0; c < 3; c++) {
+        out->n[c] = h->g.n[c];
+        out->plo[c] = h->g.plo[c];
+        out->skip[c] = h->g.skip[c];
+        out->pbc[c] = h->g.pbc[c];
+    }
+    return true;
+}
+
 int transformer_apply_scaled(const gh_transformer* h, const void* in_dev,
                              void* out_dev, int64_t nbands,
                              const double* phase_cd, double al,
