@@ -35,6 +35,7 @@ _SIGNATURES = {
     'gh_stencil_apply_shifted': (_c.c_int, [P, P, P, I64, PD, P, P, P]),
     'gh_stencil_set_tile': (_c.c_int, [P, _c.c_int, _c.c_int, _c.c_int]),
     'gh_stencil_relax': (_c.c_int, [P, _c.c_int, P, P, P, _c.c_int, D, P]),
+    'gh_stencil_relax_from': (_c.c_int, [P, P, P, P, _c.c_int, D, P]),
     'gh_stencil_batch_create': (_c.c_int, [_c.POINTER(P), _c.c_int,
                                            _c.POINTER(P), PI64, PI32, PI32,
                                            _c.c_int]),
@@ -47,6 +48,7 @@ _SIGNATURES = {
                                          _c.c_int]),
     'gh_transformer_destroy': (_c.c_int, [P]),
     'gh_transformer_apply': (_c.c_int, [P, P, P, I64, PD, P]),
+    'gh_transformer_correct': (_c.c_int, [P, P, P, P, I64, PD, P]),
     'gh_lfc_create': (_c.c_int, [_c.POINTER(P), I64, _c.c_int, PI64, PI32,
                                  PI32, PI32, PD, _c.c_int, _c.c_int, PD, D,
                                  _c.c_int]),

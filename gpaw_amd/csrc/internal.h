@@ -44,11 +44,18 @@ int stencil_rows(int dtype, const DirectStencil& h, const void* in, void* out,
 // GPAW_AMD_STENCIL names a kernel
 bool stencil_axes(const gh_stencil* h, DirectStencil* out);
 
-// Linear interpolation to the grid of half the spacing
-struct InterpGrid {
-    int n[3], plo[3], skip[3], pbc[3];   // coarse grid, ghosts below, points skipped
+// A transformer with nn = 1: input and output grid, ghosts below the input,
+// fine points skipped below (interpolation), boundaries
+struct LinearMap {
+    int n[3], m[3], plo[3], skip[3], pbc[3];
+    bool interp;
 };
-bool transformer_interp(const gh_transformer* h, int dtype, InterpGrid* out);
+bool transformer_linear(const gh_transformer* h, int dtype, LinearMap* out);
+
+// out = [base +] al * T(in) (transformers_linear.hip); base only with
+// interpolation, may be out
+int linear_map(int dtype, const LinearMap& h, const void* in, void* out, const void* base,
+               int64_t nb, const double* phase_cd, double al, hipStream_t st);
 
 // out = al * (L I u) + ga * I u + sum_q beta[q] src[q] (1 or 2 sources), I the
 // interpolation (stencil_interp.hip); GH_ERR_UNSUPPORTED where that kernel
@@ -56,6 +63,12 @@ bool transformer_interp(const gh_transformer* h, int dtype, InterpGrid* out);
 int stencil_interp(const gh_stencil* h, const gh_transformer* intp, const void* u, void* out,
                    int64_t nb, const double* phase_cd, int ns, const void* const* src,
                    const double* beta, double al, double ga, hipStream_t st);
+
+// Jacobi sweeps of a small real grid in one launch (relax_small.hip), the
+// function from f to out (may be f); out' = al * L f + ga * f + beta * s;
+// GH_ERR_UNSUPPORTED for larger grids and other stencils
+int relax_small(const gh_stencil* h, const void* f, void* out, const void* s, int sweeps,
+                double beta, double al, double ga, hipStream_t st);
 
 int device_cu_count(int* out);
 int ensure_max_lds(const void* kernel, int bytes);

@@ -1064,6 +1064,37 @@ int gh_stencil_apply_shifted(const gh_stencil* h, const void* in_dev,
                                   (hipStream_t)stream);
 }
 
+}  // extern "C"
+
+namespace {
+
+// nrelax sweeps from start (f or work) with the result in f:
+// f' = (1 - w) f + (w / c0) (s - (L f - c0 f)) = -(w / c0) L f + f + (w / c0) s
+int jacobi(const gh_stencil* h, void* start, void* f, const void* s, void* work, int nrelax,
+           double w, hipStream_t st) {
+    const double a = -w / h->diag;
+    const void* cur = start;
+    if (nrelax > 0) {
+        const int rc = relax_small(h, start, f, s, nrelax, -a, a, 1.0, st);
+        if (rc != GH_ERR_UNSUPPORTED) return rc;
+    }
+    for (int n = 0; n < nrelax; n++) {
+        void* nxt = cur == f ? work : f;
+        int rc = stencil_apply_scaled(h, cur, nxt, 1, nullptr, nullptr, s, -a, a, 1.0, st);
+        if (rc != GH_OK) return rc;
+        cur = nxt;
+    }
+    if (cur != f) {
+        const size_t bytes = (size_t)(h->n[0] * h->n[1] * h->n[2]) * dtype_size(h->dtype);
+        GH_CHECK_HIP(hipMemcpyAsync(f, cur, bytes, hipMemcpyDeviceToDevice, st));
+    }
+    return GH_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int gh_stencil_relax(const gh_stencil* h, int relax_method, void* f_dev,
                      const void* s_dev, void* work_dev, int nrelax, double w,
                      void* stream) {
@@ -1116,23 +1147,19 @@ int gh_stencil_relax(const gh_stencil* h, int relax_method, void* f_dev,
 #undef GS_SWEEPS
         return GH_OK;
     }
-    // f' = (1 - w) f + (w / c0) (s - (L f - c0 f)) = -(w / c0) L f + f + (w / c0) s
-    const double a = -w / h->diag;
-    const void* cur = f_dev;
-    void* nxt = work_dev;
-    for (int n = 0; n < nrelax; n++) {
-        int rc = gh::stencil_apply_scaled(h, cur, nxt, 1, nullptr, nullptr, s_dev,
-                                          -a, a, 1.0, st);
-        if (rc != GH_OK) return rc;
-        void* done = nxt;
-        nxt = (void*)cur;
-        cur = done;
-    }
-    if (cur != f_dev) {
-        const size_t bytes = (size_t)(h->n[0] * h->n[1] * h->n[2]) * dtype_size(h->dtype);
-        GH_CHECK_HIP(hipMemcpyAsync(f_dev, cur, bytes, hipMemcpyDeviceToDevice, st));
-    }
-    return GH_OK;
+    return jacobi(h, f_dev, f_dev, s_dev, work_dev, nrelax, w, st);
+}
+
+int gh_stencil_relax_from(const gh_stencil* h, void* f_dev, const void* s_dev, void* work_dev,
+                          int nrelax, double w, void* stream) {
+    GH_REQUIRE(h && f_dev && s_dev && work_dev, GH_ERR_ARG, "relax: null argument");
+    GH_REQUIRE(nrelax >= 0, GH_ERR_ARG, "relax: nrelax < 0");
+    GH_REQUIRE(h->dtype == GH_F64 || h->dtype == GH_F32, GH_ERR_ARG,
+               "relax: real grids only");
+    GH_REQUIRE(h->diag != 0.0, GH_ERR_ARG, "relax: zero diagonal");
+    GH_REQUIRE(f_dev != work_dev && s_dev != work_dev && f_dev != s_dev, GH_ERR_ARG,
+               "relax: f, s and work must be distinct");
+    return jacobi(h, work_dev, f_dev, s_dev, work_dev, nrelax, w, (hipStream_t)stream);
 }
 
 

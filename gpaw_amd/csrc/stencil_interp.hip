@@ -39,6 +39,7 @@
 
 #include "common.h"
 #include "internal.h"
+#include "linear_interp.h"
 
 namespace gh {
 
@@ -51,31 +52,15 @@ template <typename V> constexpr int kGhostItems = sizeof(V) > 8 ? 2 : 4;
 
 template <typename S, int R>
 struct InterpArgs {
-    int nc0, nc1, nc2;            // coarse grid
+    LinGrid<S> u;                 // coarse grid
     int n0, n1, n2;               // fine grid
-    int pbc0, pbc1, pbc2;
-    int odd0, odd1, odd2;         // zero boundaries: fine point 0 is odd
+    int odd0;                     // fine planes 2 i - odd0, + 1 belong to F_i
     int ty, lx, nyt, nxc;         // rows and coarse planes of a block
     int ncomp;                    // compute waves
     int pitch, slot;              // elements per LDS row, plane
-    int yzphase;
     S c0, k[3][R];
     S beta[2];
-    S re[3][2], im[3][2];
 };
-
-// One vector of PT fine points: where its coarse values are.
-template <int NC>
-struct Item {
-    int row[2], z[NC];            // coarse row starts, coarse z
-    unsigned flags;               // see below
-    int lds;
-};
-// flag bits: 0 fine row between two coarse rows, 1 fine z likewise (PT = 1);
-// 2, 3 row r lies beyond a zero boundary; 4.. the same for z; from 8 on two
-// bits (below, above) for each row and z that is a periodic image
-constexpr unsigned kOddY = 1, kOddZ = 2;
-constexpr unsigned zero_bits(int nc) { return 0xCu | (((1u << nc) - 1) << 4); }
 
 template <typename V, typename S, int R, int PT, bool ALIGNED, int NS>
 __global__ void __launch_bounds__(kMaxThreads)
@@ -84,15 +69,13 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
                       InterpArgs<S, R> g) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     V* lds = reinterpret_cast<V*>(smem_raw);
-    constexpr bool CPLX = is_complex<V>::value;
-    typedef S Vec __attribute__((ext_vector_type(16 / sizeof(S))));
+    typedef LinPoints<V, S, PT> Points;
+    typedef typename Points::Raw Raw;
+    typedef typename Points::Vec Vec;
     typedef Vec UVec __attribute__((aligned(sizeof(V))));
     constexpr int E = 16 / (int)sizeof(S), C = E / PT;
     static_assert(C * sizeof(S) == sizeof(V), "points per vector");
-    constexpr int NC = PT == 1 ? 2 : PT / 2 + 1;     // coarse values per row
     constexpr int NW = (R + PT - 1) / PT;            // ghost vectors per side
-    typedef Item<NC> It;
-    struct Raw { V v[2][NC]; };
 
     const int tiles = g.nyt * g.nxc;
     const int L = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -101,121 +84,12 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
     const int y0 = yt * g.ty, tye = min(g.ty, g.n1 - y0);
     const int ni = g.n0 / 2 + g.odd0;                // pairs of fine planes
     const int i0 = xc * g.lx, i1 = min(i0 + g.lx, ni);
-    const int cplane = g.nc1 * g.nc2;
-    const V* __restrict__ cb = coarse + (size_t)band * g.nc0 * cplane;
+    const V* __restrict__ cb = coarse + (size_t)band * g.u.n[0] * g.u.n[1] * g.u.n[2];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nv = (g.n2 + PT - 1) / PT;
 
-    // coarse index of a periodic image or beyond a zero boundary
-    auto wrap = [](int& c, int n, int pbc, bool& low, bool& high, bool& zero) {
-        low = c < 0;
-        high = c >= n;
-        zero = (low || high) && !pbc;
-        if (pbc) c += low ? n : high ? -n : 0;
-        else c = min(max(c, 0), n - 1);
-    };
-    auto make_item = [&](int y, int z, int ldspos) {
-        It it;
-        it.flags = 0;
-        it.lds = ldspos;
-        const int qy = y + g.odd1, cy = (qy >> 1) - g.odd1;
-        if (qy & 1) it.flags |= kOddY;
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            int c = cy + ((qy & 1) ? r : 0);
-            bool low, high, zero;
-            wrap(c, g.nc1, g.pbc1, low, high, zero);
-            it.row[r] = c * g.nc2;
-            if (zero) it.flags |= 4u << r;
-            it.flags |= (unsigned)low << (8 + 2 * r) | (unsigned)high << (9 + 2 * r);
-        }
-        const int qz = z + g.odd2, cz = (qz >> 1) - g.odd2;
-        if (PT == 1 && (qz & 1)) it.flags |= kOddZ;
-#pragma unroll
-        for (int k = 0; k < NC; k++) {
-            int c = cz + (PT == 1 && !(qz & 1) ? 0 : k);
-            bool low, high, zero;
-            wrap(c, g.nc2, g.pbc2, low, high, zero);
-            it.z[k] = c;
-            if (zero) it.flags |= 16u << k;
-            it.flags |= (unsigned)low << (12 + 2 * k) | (unsigned)high << (13 + 2 * k);
-        }
-        return it;
-    };
-    // coarse plane of F_i: its image inside the grid
-    auto plane_ptr = [&](int i) {
-        int c = i - g.odd0;
-        if (g.pbc0) c += c < 0 ? g.nc0 : c >= g.nc0 ? -g.nc0 : 0;
-        else c = min(max(c, 0), g.nc0 - 1);
-        return cb + (size_t)c * cplane;
-    };
-    auto load = [&](const It& it, int i, Raw& raw) {
-        const V* p = plane_ptr(i);
-#pragma unroll
-        for (int r = 0; r < 2; r++)
-#pragma unroll
-            for (int k = 0; k < NC; k++) raw.v[r][k] = p[it.row[r] + it.z[k]];
-    };
-    const bool zeros = !(g.pbc1 && g.pbc2);
-    auto half = [](V a, V b) { return vscale(vadd(a, b), (S)0.5); };
-    // F_i at the item's points
-    auto make = [&](const It& it, int i, Raw raw) {
-        if (zeros && __any((int)(it.flags & zero_bits(NC)))) {
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int k = 0; k < NC; k++)
-                    if (it.flags & (4u << r | 16u << k)) raw.v[r][k] = vzero<V>();
-        }
-        if constexpr (CPLX) {
-            if (g.yzphase && __any((int)(it.flags >> 8))) {
-#pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    const bool l = it.flags >> (8 + 2 * r) & 1, h = it.flags >> (9 + 2 * r) & 1;
-                    const S pr = l ? g.re[1][1] : h ? g.re[1][0] : (S)1;
-                    const S pi = l ? g.im[1][1] : h ? g.im[1][0] : (S)0;
-#pragma unroll
-                    for (int k = 0; k < NC; k++) {
-                        const bool zl = it.flags >> (12 + 2 * k) & 1,
-                                   zh = it.flags >> (13 + 2 * k) & 1;
-                        raw.v[r][k] = mul_phase(raw.v[r][k], pr, pi);
-                        raw.v[r][k] = mul_phase(raw.v[r][k],
-                                                zl ? g.re[2][1] : zh ? g.re[2][0] : (S)1,
-                                                zl ? g.im[2][1] : zh ? g.im[2][0] : (S)0);
-                    }
-                }
-            }
-        }
-        V f[2][PT];
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            if constexpr (PT == 1) {
-                f[r][0] = it.flags & kOddZ ? half(raw.v[r][0], raw.v[r][1]) : raw.v[r][0];
-            } else {
-#pragma unroll
-                for (int e = 0; e < PT; e += 2) {
-                    const V m = half(raw.v[r][e / 2], raw.v[r][e / 2 + 1]);
-                    f[r][e] = g.odd2 ? m : raw.v[r][e / 2];
-                    f[r][e + 1] = g.odd2 ? raw.v[r][e / 2 + 1] : m;
-                }
-            }
-        }
-        V o[PT];
-        const int c = i - g.odd0;
-        const bool xlow = c < 0, xhigh = c >= g.nc0;
-#pragma unroll
-        for (int e = 0; e < PT; e++) {
-            o[e] = it.flags & kOddY ? half(f[0][e], f[1][e]) : f[0][e];
-            if (!g.pbc0 && (xlow || xhigh)) o[e] = vzero<V>();
-            if constexpr (CPLX)
-                if (xlow || xhigh) o[e] = mul_phase(o[e], g.re[0][xlow], g.im[0][xlow]);
-        }
-        Vec v;
-        __builtin_memcpy(&v, o, sizeof(v));
-        return v;
-    };
-    auto put = [&](const It& it, int i, Vec v) {
-        *reinterpret_cast<Vec*>(lds + (i & 1) * g.slot + it.lds) = v;
+    auto put = [&](int pos, int i, Vec v) {
+        *reinterpret_cast<Vec*>(lds + (i & 1) * g.slot + pos) = v;
     };
 
     if (wave >= g.ncomp) {
@@ -224,7 +98,8 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
         const int rowvec = nv + 2 * NW;                       // vectors per LDS row
         const int nrow = 2 * R * rowvec, n = nrow + tye * 2 * NW;
         constexpr int GI = kGhostItems<V>;
-        It it[GI];
+        Points it[GI];
+        int pos[GI];
         Raw raw[GI];
 #pragma unroll
         for (int a = 0; a < GI; a++) {
@@ -240,15 +115,16 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
                 if (c >= NW) c += nv;
                 r += R;
             }
-            it[a] = make_item(y0 - R + r, (c - NW) * PT, r * g.pitch + c * PT);
+            it[a].set(y0 - R + r, (c - NW) * PT, g.u);
+            pos[a] = r * g.pitch + c * PT;
         }
         auto all = [&](int i) {
 #pragma unroll
-            for (int a = 0; a < GI; a++) load(it[a], i, raw[a]);
+            for (int a = 0; a < GI; a++) it[a].load(cb, i, g.u, raw[a]);
         };
         auto store = [&](int i) {
 #pragma unroll
-            for (int a = 0; a < GI; a++) put(it[a], i, make(it[a], i, raw[a]));
+            for (int a = 0; a < GI; a++) put(pos[a], i, it[a].make(raw[a], i, g.u));
         };
         all(i0);
         store(i0);
@@ -269,7 +145,9 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
     // same places), so that no access is conditional
     const int pp = min((int)threadIdx.x, tye * nv - 1);
     const int yl = pp / nv, z = (pp - yl * nv) * PT;
-    const It it = make_item(y0 + yl, z, (yl + R) * g.pitch + (NW * PT + z));
+    Points it;
+    it.set(y0 + yl, z, g.u);
+    const int pos = (yl + R) * g.pitch + (NW * PT + z);
     const bool part = !ALIGNED && z + PT > g.n2;
     const int short_by = ALIGNED ? 0 : nv * PT - g.n2;
     const int down = part ? short_by : 0;
@@ -295,7 +173,7 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
     };
     // y and z parts and the centre on the plane of F_i (f: its own points)
     auto yz_part = [&](int i, Vec f) {
-        const V* p = lds + (i & 1) * g.slot + it.lds;
+        const V* p = lds + (i & 1) * g.slot + pos;
         Vec acc = f * g.c0;
 #pragma unroll
         for (int j = 0; j < R; j++)
@@ -333,14 +211,14 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
     {
         Raw r[4];
 #pragma unroll
-        for (int a = 0; a < 4; a++) load(it, i0 - 2 + a, r[a]);
+        for (int a = 0; a < 4; a++) it.load(cb, i0 - 2 + a, g.u, r[a]);
 #pragma unroll
-        for (int a = 0; a < 4; a++) f[a] = make(it, i0 - 2 + a, r[a]);
+        for (int a = 0; a < 4; a++) f[a] = it.make(r[a], i0 - 2 + a, g.u);
     }
-    put(it, i0, f[2]);
-    put(it, i0 + 1, f[3]);
+    put(pos, i0, f[2]);
+    put(pos, i0 + 1, f[3]);
     Raw raw;
-    load(it, i0 + 2, raw);
+    it.load(cb, i0 + 2, g.u, raw);
     Vec s[2][NS];
     auto load_src = [&](int i, Vec (&t)[2][NS]) {
 #pragma unroll
@@ -356,9 +234,9 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
     Vec w0 = yz_part(i0, f[2]);
     for (int i = i0; i < i1; i++) {
         __syncthreads();
-        f[4] = make(it, i + 2, raw);
-        put(it, i + 2, f[4]);
-        load(it, i + 3, raw);
+        f[4] = it.make(raw, i + 2, g.u);
+        put(pos, i + 2, f[4]);
+        it.load(cb, i + 3, g.u, raw);
         Vec t[2][NS];
         if (kAhead) load_src(i + 1, t);
         else load_src(i, s);
@@ -391,21 +269,22 @@ stencil_interp_kernel(const V* __restrict__ coarse, V* __restrict__ out,
 }
 
 template <typename V, typename S, int R>
-int launch_r(const DirectStencil& h, const InterpGrid& ig, const void* coarse, void* out,
+int launch_r(const DirectStencil& h, const LinearMap& ig, const void* coarse, void* out,
              int64_t nbands, const double* phase_cd, int ns, const void* const* src,
              const double* beta, double alpha, double gamma, hipStream_t st) {
     constexpr int PT = 16 / (int)sizeof(V), NW = (R + PT - 1) / PT;
     InterpArgs<S, R> g;
-    g.nc0 = ig.n[0]; g.nc1 = ig.n[1]; g.nc2 = ig.n[2];
     g.n0 = h.n[0]; g.n1 = h.n[1]; g.n2 = h.n[2];
-    g.pbc0 = h.pbc[0]; g.pbc1 = h.pbc[1]; g.pbc2 = h.pbc[2];
-    g.odd0 = !g.pbc0; g.odd1 = !g.pbc1; g.odd2 = !g.pbc2;
+    g.odd0 = !h.pbc[0];
     for (int c = 0; c < 3; c++) {
         // the two grids of a V-cycle; an image is one period away at most
         const int odd = !h.pbc[c];
         if (ig.pbc[c] != h.pbc[c] || ig.plo[c] != odd || ig.skip[c] != odd ||
             h.n[c] != 2 * ig.n[c] + odd || ig.n[c] < 4)
             return GH_ERR_UNSUPPORTED;
+        g.u.n[c] = ig.n[c];
+        g.u.pbc[c] = ig.pbc[c];
+        g.u.plo[c] = g.u.skip[c] = odd;
         for (int j = 0; j < R; j++) {
             if (h.cm[c][j] != h.cp[c][j]) return GH_ERR_UNSUPPORTED;
             g.k[c][j] = (S)(alpha * h.cm[c][j]);
@@ -414,21 +293,14 @@ int launch_r(const DirectStencil& h, const InterpGrid& ig, const void* coarse, v
     // two sources: the 7-point Laplacians of the coarse levels
     if (ns == 2 && R != 1) return GH_ERR_UNSUPPORTED;
     // a vector that straddles the end of a periodic row has no place here
-    if (g.pbc2 && g.n2 % PT) return GH_ERR_UNSUPPORTED;
+    if (h.pbc[2] && g.n2 % PT) return GH_ERR_UNSUPPORTED;
     uintptr_t bits = (uintptr_t)coarse | (uintptr_t)out;
     for (int q = 0; q < ns; q++) bits |= (uintptr_t)src[q];
     if (bits & (sizeof(S) - 1)) return GH_ERR_UNSUPPORTED;
     g.c0 = (S)(alpha * h.c0 + gamma);
     g.beta[0] = (S)beta[0];
     g.beta[1] = ns > 1 ? (S)beta[1] : (S)0;
-    const Phases ph = make_phases(phase_cd);
-    g.yzphase = 0;
-    for (int c = 0; c < 3; c++)
-        for (int d = 0; d < 2; d++) {
-            g.re[c][d] = (S)ph.re[c][d];
-            g.im[c][d] = (S)ph.im[c][d];
-            if (c > 0 && (g.re[c][d] != (S)1 || g.im[c][d] != (S)0)) g.yzphase = 1;
-        }
+    set_phases(g.u, phase_cd);
     const int nv = (g.n2 + PT - 1) / PT, ni = g.n0 / 2 + g.odd0;
     g.pitch = (nv + 2 * NW) * PT;
     auto lds_of = [&](int ty) { return 2 * (size_t)(ty + 2 * R) * g.pitch * sizeof(V); };
@@ -492,7 +364,7 @@ int launch_r(const DirectStencil& h, const InterpGrid& ig, const void* coarse, v
 }
 
 template <typename V, typename S>
-int launch(const DirectStencil& h, const InterpGrid& ig, const void* u, void* out, int64_t nb,
+int launch(const DirectStencil& h, const LinearMap& ig, const void* u, void* out, int64_t nb,
            const double* ph, int ns, const void* const* src, const double* beta, double al,
            double ga, hipStream_t st) {
     switch (h.R) {
@@ -509,9 +381,9 @@ int stencil_interp(const gh_stencil* h, const gh_transformer* intp, const void* 
                    int64_t nb, const double* ph, int ns, const void* const* src,
                    const double* beta, double al, double ga, hipStream_t st) {
     DirectStencil d;
-    InterpGrid ig;
+    LinearMap ig;
     const int dtype = stencil_dtype(h);
-    if (!stencil_axes(h, &d) || !transformer_interp(intp, dtype, &ig)) return GH_ERR_UNSUPPORTED;
+    if (!stencil_axes(h, &d) || !transformer_linear(intp, dtype, &ig) || !ig.interp) return GH_ERR_UNSUPPORTED;
     switch (dtype) {
         case GH_F64: return launch<double, double>(d, ig, u, out, nb, ph, ns, src, beta, al, ga, st);
         case GH_C128: return launch<cplx<double>, double>(d, ig, u, out, nb, ph, ns, src, beta, al, ga, st);

@@ -17,7 +17,9 @@
 // along x.  For every input plane it needs, the block stages the input rows
 // of its tile in LDS, filters them along z (LDS -> LDS) and along y (LDS ->
 // registers), and keeps the last 2K-1 (restrict) or K (interpolate) filtered
-// planes in a register queue that the x-filter reads.
+// planes in a register queue that the x-filter reads.  The short filter
+// (nn = 1) comes here only for restrictions of many real functions, see
+// staged(); its other calls run in transformers_linear.hip.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -621,8 +623,7 @@ constexpr int ppt_of(bool interp) {
 // what the CUs hold go into further rounds.  Cutting the runs until 2048
 // blocks existed, as before, primed 9 to 11 planes for every 8: 2 densities
 // 112^3 -> 224^3 with nn = 3 took 119 us and take 60, 128 complex64 functions
-// restricted from 112^3 with nn = 3 684 and 520 us, 16 FP32 functions 48^3 with
-// nn = 1 14.6 and 8.2 us.
+// restricted from 112^3 with nn = 3 684 and 520 us.
 struct TTile {
     int tj = 0, lx = 0, nry = 0;
     size_t lds = 0;
@@ -700,7 +701,13 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
     for (int c = 1; c < 3; c++)
         for (int d = 0; d < 2; d++)
             if (ph.re[c][d] != (S)1 || ph.im[c][d] != (S)0) g.yz_trivial = 0;
-    if (h->interp)
+    if constexpr (K == 2) {
+        // the short filter's interpolation and its other restrictions:
+        // transformers_linear.hip
+        constexpr int VEC = 16 / sizeof(V);
+        hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R, VEC>), dim3((unsigned)nblocks),
+                           dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
+    } else if (h->interp)
         hipLaunchKernelGGL((interpolate_kernel<V, S, K, PPT_I>), dim3((unsigned)nblocks),
                            dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
     else if (constexpr int VEC = 16 / sizeof(V);
@@ -719,7 +726,9 @@ template <typename V, typename S>
 int launch_k(const gh_transformer* h, const void* in, void* out, int64_t nb,
              const double* ph, double al, hipStream_t st) {
     switch (h->nn) {
-        case 1: return launch_t<V, S, 2>(h, in, out, nb, ph, al, st);
+        case 1:
+            if constexpr (!is_complex<V>::value) return launch_t<V, S, 2>(h, in, out, nb, ph, al, st);
+            break;
         case 2: return launch_t<V, S, 4>(h, in, out, nb, ph, al, st);
         case 3: return launch_t<V, S, 6>(h, in, out, nb, ph, al, st);
         case 4: return launch_t<V, S, 8>(h, in, out, nb, ph, al, st);
@@ -729,6 +738,12 @@ int launch_k(const gh_transformer* h, const void* in, void* out, int64_t nb,
 }
 
 }  // namespace
+
+namespace gh {
+namespace {
+bool lin_rows_fit(const gh_transformer* h);
+}
+}  // namespace gh
 
 extern "C" {
 
@@ -815,6 +830,22 @@ int gh_transformer_apply(const gh_transformer* h, const void* in_dev,
                                         1.0, (hipStream_t)stream);
 }
 
+int gh_transformer_correct(const gh_transformer* h, const void* in_dev, const void* base_dev,
+                           void* out_dev, int64_t nbands, const double* phase_cd,
+                           void* stream) {
+    GH_REQUIRE(h, GH_ERR_ARG, "transformer_correct: null handle");
+    GH_REQUIRE(nbands >= 0, GH_ERR_ARG, "transformer_correct: nbands < 0");
+    gh::LinearMap lin;
+    GH_REQUIRE(gh::transformer_linear(h, h->dtype, &lin) && h->interp && lin_rows_fit(h),
+               GH_ERR_UNSUPPORTED, "transformer_correct: interpolation with nn = 1 only");
+    if (nbands == 0) return GH_OK;  // empty arrays may carry null pointers
+    GH_REQUIRE(in_dev && base_dev && out_dev, GH_ERR_ARG, "transformer_correct: null argument");
+    GH_REQUIRE(in_dev != out_dev && in_dev != base_dev, GH_ERR_ARG,
+               "transformer_correct: in must differ from base and out");
+    return gh::linear_map(h->dtype, lin, in_dev, out_dev, base_dev, nbands, phase_cd, -1.0,
+                          (hipStream_t)stream);
+}
+
 }  // extern "C"
 
 namespace gh {
@@ -826,14 +857,40 @@ int64_t transformer_out_points(const gh_transformer* h) {
     return (int64_t)h->g.m[0] * h->g.m[1] * h->g.m[2];
 }
 
-bool transformer_interp(const gh_transformer* h, int dtype, InterpGrid* out) {
-    if (!h->interp || h->nn != 1 || h->dtype != dtype) return false;
+namespace {
+
+// Restriction with the short filter of many real functions whose rows are
+// whole 16-byte vectors: beyond the 256 MB of the last-level cache the staged
+// kernel's single read of the input wins.  FP64, 16 x 112^3 (22 M points)
+// staged 36.3 us, not staged 35.3; 200 x 64^3 (52 M) 107 and 132; FP32, 64 x
+// 64^3 (17 M) 20.8 and 21.1, 256 x 64^3 68 and 105.  Complex data gain from
+// it nowhere (complex64, 200 x 64^3, k along x 147 and 139).
+bool staged(const gh_transformer* h, const void* in, int64_t nbands) {
+    return !h->interp && (h->dtype == GH_F64 || h->dtype == GH_F32) &&
+           h->g.vec == 16 / dtype_size(h->dtype) && ((uintptr_t)in & 15u) == 0 &&
+           nbands * transformer_in_points(h) > 24000000;
+}
+
+// Rows longer than a block of the staged kernels are refused for every filter.
+bool lin_rows_fit(const gh_transformer* h) {
+    const TGeom& g = h->g;
+    const int vs = dtype_size(h->dtype), ppt = h->interp || vs <= 8 ? 2 : 1;
+    const size_t lds = h->interp ? (size_t)4 * (g.zw + g.m[2]) * vs : (size_t)4 * g.zw * vs;
+    return lds <= 64 * 1024 && g.m[2] <= 1024 * ppt;
+}
+
+}  // namespace
+
+bool transformer_linear(const gh_transformer* h, int dtype, LinearMap* out) {
+    if (h->nn != 1 || h->dtype != dtype) return false;
     for (int c = 0; c < 3; c++) {
         out->n[c] = h->g.n[c];
+        out->m[c] = h->g.m[c];
         out->plo[c] = h->g.plo[c];
         out->skip[c] = h->g.skip[c];
         out->pbc[c] = h->g.pbc[c];
     }
+    out->interp = h->interp;
     return true;
 }
 
@@ -846,6 +903,12 @@ int transformer_apply_scaled(const gh_transformer* h, const void* in_dev,
     if (nbands == 0) return GH_OK;  // empty arrays may carry null pointers
     GH_REQUIRE(in_dev && out_dev, GH_ERR_ARG, "transformer_apply: null argument");
     GH_REQUIRE(in_dev != out_dev, GH_ERR_ARG, "transformer_apply: in and out must differ");
+    LinearMap lin;
+    if (transformer_linear(h, h->dtype, &lin) && !staged(h, in_dev, nbands)) {
+        GH_REQUIRE(lin_rows_fit(h), GH_ERR_UNSUPPORTED,
+                   "transformer: grid rows too long for one block");
+        return linear_map(h->dtype, lin, in_dev, out_dev, nullptr, nbands, phase_cd, al, st);
+    }
     switch (h->dtype) {
         case GH_F64: return launch_k<double, double>(h, in_dev, out_dev, nbands, phase_cd, al, st);
         case GH_C128: return launch_k<cplx<double>, double>(h, in_dev, out_dev, nbands, phase_cd, al, st);

@@ -160,6 +160,16 @@ class FDOperator:
                 self.handle, int(relax_method), f.data_ptr(), s.data_ptr(),
                 self._work.data_ptr(), int(n), w, stream_ptr()))
 
+    def _relax_from(self, f_g, s_g, work_g, n, w):
+        """n Jacobi sweeps that start from work_g and end in f_g (an odd
+        number of them needs no copy)."""
+        with Staged(f_g, writeback=True, dtype=self.dtype) as f, \
+                Staged(s_g, dtype=self.dtype) as s, \
+                Staged(work_g, dtype=self.dtype) as work:
+            _lib.check(self._lib.gh_stencil_relax_from(
+                self.handle, f.data_ptr(), s.data_ptr(), work.data_ptr(),
+                int(n), float(w), stream_ptr()))
+
     def get_diagonal_element(self):
         return self._lib.gh_stencil_diagonal(self.handle)
 

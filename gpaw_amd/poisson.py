@@ -364,10 +364,20 @@ class FDPoissonSolver:
             self.restrictors[level].apply(residual, self.rhos[level + 1])
             self.phis[level + 1].zero_()
             self._cycle(4.0 * step, level + 1)
-            self.interpolators[level].apply(self.phis[level + 1], residual)
-            self.phis[level] -= residual
-        op.relax(self.relax_method, self.phis[level], self.rhos[level],
-                 self.postsmooths[level], self.weights[level])
+            # an odd number of Jacobi sweeps starts from the corrected
+            # potential in the residual's array and ends in phi
+            odd = self.relax_method == 2 and self.postsmooths[level] % 2 == 1
+            self.interpolators[level]._subtract(
+                self.phis[level + 1], self.phis[level],
+                residual if odd else self.phis[level])
+        else:
+            odd = False
+        if odd:
+            op._relax_from(self.phis[level], self.rhos[level], residual,
+                           self.postsmooths[level], self.weights[level])
+        else:
+            op.relax(self.relax_method, self.phis[level], self.rhos[level],
+                     self.postsmooths[level], self.weights[level])
         if level == 0:
             op.apply(self.phis[0][None], residual[None],
                      src_xg=self.rhos[0][None], beta=-1.0)

@@ -87,6 +87,16 @@ class _Transformer:
                 stream_ptr()))
         return output
 
+    def _subtract(self, input, base, output):
+        """output = base - T(input) for one grid (interpolation with nn = 1;
+        output may be base)."""
+        with Staged(input, dtype=self.dtype) as a, \
+                Staged(base, dtype=self.dtype) as b, \
+                Staged(output, dtype=self.dtype) as c:
+            _lib.check(self._lib.gh_transformer_correct(
+                self.handle, a.data_ptr(), b.data_ptr(), c.data_ptr(), 1, None,
+                stream_ptr()))
+
 
 def Transformer(gdin, gdout, nn=1, dtype=float, xp=None):
     if nn != 9:

@@ -115,6 +115,11 @@ int gh_stencil_relax(const gh_stencil* h, int relax_method, void* f_dev,
                      const void* s_dev, void* work_dev, int nrelax, double w,
                      void* stream);
 
+/* As gh_stencil_relax with relax_method 2, but the sweeps start from the
+ * function in work_dev (overwritten) and end in f_dev. */
+int gh_stencil_relax_from(const gh_stencil* h, void* f_dev, const void* s_dev,
+                          void* work_dev, int nrelax, double w, void* stream);
+
 /* ------------------------------------------------------ batched cells --
  * Several independent grids ("cells") of different sizes and band counts in
  * one persistent launch of the LDS-ring stencil: out_c = L_c in_c
@@ -164,6 +169,12 @@ int gh_transformer_destroy(gh_transformer* h);
 int gh_transformer_apply(const gh_transformer* h, const void* in_dev,
                          void* out_dev, int64_t nbands,
                          const double* phase_cd, void* stream);
+
+/* out = base - T(in) for an interpolation with nn = 1 (another transformer:
+ * GH_ERR_UNSUPPORTED); base_dev may be out_dev. */
+int gh_transformer_correct(const gh_transformer* h, const void* in_dev,
+                           const void* base_dev, void* out_dev, int64_t nbands,
+                           const double* phase_cd, void* stream);
 
 /* ----------------------------------------------------------------- LFC --
  * Replaces cgpaw.LFC (reference c/lfc.c:146-257, built by lfc.py:273-369)
