@@ -74,6 +74,7 @@ _SIGNATURES = {
     'gh_multi_lincomb': (_c.c_int, [_c.c_int, I64, I64, _c.c_int,
                                     _c.POINTER(P), P, P, P]),
     'gh_gram_work_bytes': (I64, [_c.c_int, I64, I64, I64, _c.c_int]),
+    'gh_rotate': (_c.c_int, [_c.c_int, _c.c_int, I64, P, P, P, P]),
     'gh_gram': (_c.c_int, [_c.c_int, I64, I64, I64, P, I64, P, I64, D,
                            _c.c_int, _c.c_int, P, P, I64, P]),
     'gh_unet_conv3_weight_elems': (I64, [_c.c_int, _c.c_int]),

@@ -65,8 +65,8 @@ class Eigensolver:
             H = 0.5 * (H + H.conj().T)
         eps, C = torch.linalg.eigh(H)
         U = C.T.contiguous().to(psi.dtype)   # rotations in the data precision
-        wfs.psit = (U @ psi).reshape(psit.shape)
-        Htpsit = (U @ hpsi).reshape(psit.shape)
+        wfs.psit = blas.rotate(U, psi).reshape(psit.shape)
+        Htpsit = blas.rotate(U, hpsi).reshape(psit.shape)
         if P is not None:
             wfs.P = U @ P
         wfs.eps = eps.to(torch.float64).contiguous()

@@ -87,7 +87,7 @@ class FDWaveFunctions:
         Linv = Linv.to(psi.dtype)   # the rotation in the data precision
         # the rotated wave functions go to a new buffer (no copy back):
         # psit is re-bound, as is every rotation below
-        self.psit = (Linv @ psi).reshape(self.psit.shape)
+        self.psit = blas.rotate(Linv, psi).reshape(self.psit.shape)
         if self.P is not None:
             self.P = Linv @ self.P
         self.orthonormalized = True

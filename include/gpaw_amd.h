@@ -344,6 +344,11 @@ int gh_multi_lincomb(int dtype, int64_t nbands, int64_t n, int k,
 int gh_add_to_density(int dtype, int64_t nbands, int64_t n, const double* f_dev,
                       const void* psit_dev, double* nt_dev, void* stream);
 
+/* out = U psi: U (m, k), psi (k, n), out (m, n), row-major FP64, m and k at
+ * most 64, n below 2^27 (more: GH_ERR_UNSUPPORTED). */
+int gh_rotate(int m, int k, int64_t n, const double* U_dev, const double* psi_dev,
+              double* out_dev, void* stream);
+
 /* ------------------------------------------------- band overlap matrices --
  * Replaces the rk / r2k / mmm(..., 'N', ..., 'C') contractions of
  * gpaw/utilities/blas.py:39,273,314 (c/blas.c:48,101,140) as used for the

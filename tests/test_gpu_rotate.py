@@ -1,0 +1,34 @@
+"""Rotation of wave functions at the edges of its 16 x 16 x 4 tiles and at
+the largest sizes, against a product in FP64 on the CPU; infinities stay in
+the rows of the functions that hold them."""
+import pytest
+
+torch = pytest.importorskip('torch')
+pytestmark = pytest.mark.gpu
+
+from gpaw_amd import blas  # noqa: E402
+
+
+# k products of order one: k roundings of 1.1e-16 of at most k
+@pytest.mark.parametrize('m,k', [(1, 1), (3, 5), (16, 16), (17, 15), (48, 33),
+                                 (64, 64), (10, 64), (64, 1), (65, 64)])
+@pytest.mark.parametrize('n', [1, 15, 17, 4096 * 16 + 3])
+def test_rotate(m, k, n):
+    g = torch.Generator().manual_seed(m * 100 + k)
+    U = torch.randn(m, k, generator=g, dtype=torch.float64)
+    psi = torch.randn(k, n, generator=g, dtype=torch.float64)
+    out = blas.rotate(U.cuda(), psi.cuda()).cpu()
+    want = U @ psi
+    assert out.shape == want.shape
+    assert (out - want).abs().max() <= 1.1e-16 * k * (k + 12)
+
+
+def test_transposed_and_infinite():
+    g = torch.Generator().manual_seed(7)
+    U = torch.randn(20, 30, generator=g, dtype=torch.float64)
+    psi = torch.randn(20, 50, generator=g, dtype=torch.float64)
+    psi[19, 7] = float('inf')
+    out = blas.rotate(U.T.cuda(), psi.cuda()).cpu()
+    want = U.T @ psi
+    assert torch.equal(torch.isinf(out), torch.isinf(want))
+    assert bool((torch.isinf(out).sum(0) == 30 * (torch.arange(50) == 7)).all())
