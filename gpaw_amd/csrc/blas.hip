@@ -18,7 +18,9 @@
 //   7. u1 = t1 - 4s (L1 t1 - r1)               (= d1 after step 11)
 //   8. d0' = -I1(u1)                           (step 12)
 //   9. d0 = s (L0 d0' - R) - d0'               (steps 13-14)
-// Nine kernels in place of the reference's twenty array passes.
+// Steps 5-7 and 8-9 are one kernel each (stencil_interp.hip; where it has no
+// path, the steps as listed): six kernels in place of the reference's twenty
+// array passes.
 #include <algorithm>
 #include <mutex>
 

@@ -617,19 +617,23 @@ constexpr int ppt_of(bool interp) {
 
 // Tile (output rows) and x-run of a block: the pair with the least estimated
 // time.  A block walks its run's input planes (the first ones only prime the
-// filter queue); a plane costs two barriers and their latency, about the time
-// of 6 KB at a CU's share of the HBM rate, plus what every block beside it on
-// the CU moves through HBM and, at a fifteenth, through LDS.  Blocks beyond
-// what the CUs hold go into further rounds.  Cutting the runs until 2048
-// blocks existed, as before, primed 9 to 11 planes for every 8: 2 densities
-// 112^3 -> 224^3 with nn = 3 took 119 us and take 60, 128 complex64 functions
-// restricted from 112^3 with nn = 3 684 and 520 us.
+// filter queue).  A plane costs what every block beside it on the CU moves
+// through HBM and, at a fifteenth, through LDS, or, if that is longer, the
+// latency of its two barriers and its loads: 0.8 us (restriction) or 1.6
+// (interpolation) and 0.17 per load of a thread, four times that where every
+// element's phase is worked out; in bytes at a CU's share of the HBM rate
+// (20 KB per us).  Blocks beyond what the CUs hold go into further rounds.
+// Cutting the runs until 2048 blocks existed, as before, primed 9 to 11
+// planes for every 8: 2 densities 112^3 -> 224^3 with nn = 3 took 119 us and
+// take 61, 128 complex64 functions restricted from 112^3 684 and 520 us, 3 of
+// 46 x 40 x 44 with a general k 69 and 44.
 struct TTile {
     int tj = 0, lx = 0, nry = 0;
     size_t lds = 0;
 };
 
-TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, int ncu) {
+TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, bool phases,
+                  int ncu) {
     const TGeom& g = h->g;
     const int K = 2 * h->nn;
     TTile best;
@@ -649,6 +653,8 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, i
         const double taps = h->interp ? (K + 2) / 2.0 * (nry * g.m[2] + tj * g.m[2])
                                       : (K + 2.0) * (tj * g.zw + tj * g.m[2]);
         const double plane = hbm + taps * vsize / 15;
+        const double loads = std::ceil((double)nry * g.zw / (h->interp ? 1 : g.vec) / thr);
+        const double fixed = (h->interp ? 32e3 : 16e3) + 3.4e3 * loads * (phases ? 4 : 1);
         const double room = (double)ncu * fit;
         // steps of an eighth: a few microseconds per call for this search
         for (int nxc = 1; nxc <= std::max(1, g.m[0] / 2); nxc += 1 + nxc / 8) {
@@ -657,7 +663,8 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, i
             const double rounds = std::ceil(blocks / room);
             const double beside = std::min((double)fit, std::ceil(blocks / ncu));
             const double planes = h->interp ? (lx + 1) / 2 + K - 1 : 2 * lx + 2 * K - 3;
-            const double t = rounds * planes * (beside * plane + 6144.0);
+            const double bytes = beside * plane;
+            const double t = rounds * planes * (std::max(bytes, fixed) + 0.2 * std::min(bytes, fixed));
             if (best.tj == 0 || t < tbest) {
                 tbest = t;
                 best.tj = tj;
@@ -682,7 +689,13 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
     int ncu = 0;
     const int crc = device_cu_count(&ncu);
     if (crc != GH_OK) return crc;
-    const TTile tile = choose_tile(h, sizeof(V), ppt, nbands, ncu);
+    TPhase<S> ph = tphase<S>(phase_cd);
+    g.yz_trivial = 1;
+    for (int c = 1; c < 3; c++)
+        for (int d = 0; d < 2; d++)
+            if (ph.re[c][d] != (S)1 || ph.im[c][d] != (S)0) g.yz_trivial = 0;
+    const TTile tile = choose_tile(h, sizeof(V), ppt, nbands,
+                                   is_complex<V>::value && !g.yz_trivial, ncu);
     GH_REQUIRE(tile.tj > 0, GH_ERR_UNSUPPORTED,
                "transformer: grid rows too long for one block");
     const int tj = tile.tj;
@@ -696,11 +709,6 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
     thr = ((thr + 63) / 64) * 64;
     int64_t nblocks = nbands * (int64_t)g.nyt * g.nxc;
     GH_REQUIRE(nblocks < (1ll << 31), GH_ERR_SHAPE, "transformer: too many blocks");
-    TPhase<S> ph = tphase<S>(phase_cd);
-    g.yz_trivial = 1;
-    for (int c = 1; c < 3; c++)
-        for (int d = 0; d < 2; d++)
-            if (ph.re[c][d] != (S)1 || ph.im[c][d] != (S)0) g.yz_trivial = 0;
     if constexpr (K == 2) {
         // the short filter's interpolation and its other restrictions:
         // transformers_linear.hip
