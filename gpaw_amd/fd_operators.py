@@ -175,7 +175,7 @@ class FDOperator:
 
     def set_tile(self, rows=0, planes=0, depth=0):
         """Tile shape of the stencil kernel: rows per block, x-planes per
-        block, prefetch depth (0 = automatic)."""
+        block, prefetch depth of batched cells (0 = automatic)."""
         _lib.check(self._lib.gh_stencil_set_tile(self.handle, int(rows),
                                                  int(planes), int(depth)))
 

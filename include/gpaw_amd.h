@@ -101,8 +101,9 @@ int gh_stencil_apply_shifted(const gh_stencil* h, const void* in_dev,
                              const double* eps_dev, void* stream);
 
 /* Tile choice of the stencil kernel: rows of the (y, z) tile per block,
- * planes per block along x, and the prefetch depth in planes (2 or 3) of
- * the LDS-ring kernel; 0 = automatic.  Used by the autotuner. */
+ * planes per block along x; 0 = automatic.  depth: prefetch depth in planes
+ * (2 or 3) of batched cells, without effect on a single grid.  Used by the
+ * autotuner. */
 int gh_stencil_set_tile(gh_stencil* h, int rows, int planes, int depth);
 
 /* Jacobi relaxation of L f = s in place (replaces Operator.relax,
@@ -110,7 +111,8 @@ int gh_stencil_set_tile(gh_stencil* h, int rows, int planes, int depth);
  *   f <- (1 - w) f + w (s - sum_{c != 0} coef_c f[shift_c]) / coef_0
  * with the boundary conditions of gh_stencil_apply (no Bloch phases).
  * One real grid (n0, n1, n2); work_dev: a device array of the same size.
- * relax_method 1 (Gauss-Seidel) returns GH_ERR_UNSUPPORTED. */
+ * relax_method 1: Gauss-Seidel sweeps in C order, stencils along the grid
+ * axes only. */
 int gh_stencil_relax(const gh_stencil* h, int relax_method, void* f_dev,
                      const void* s_dev, void* work_dev, int nrelax, double w,
                      void* stream);
