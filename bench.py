@@ -833,7 +833,7 @@ def main():
                      'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
                      'frac': round(achieved / HBM_PEAK_GBS, 4),
                      'traffic': STENCIL_TRAFFIC_BYTES.get((N, nb)),
-                     'kernel': 'stencil_ring_kernel<double,R=3,V> '
+                     'kernel': 'stencil_rows_kernel<double,R=3,V> '
                                '(T psi + V psi, one pass)',
                      'kernel_ms': round(stencil_ms, 4),
                      'traffic_GBps': (round(STENCIL_TRAFFIC_BYTES[(N, nb)] /

@@ -18,8 +18,8 @@
 // of its tile in LDS, filters them along z (LDS -> LDS) and along y (LDS ->
 // registers), and keeps the last 2K-1 (restrict) or K (interpolate) filtered
 // planes in a register queue that the x-filter reads.  The short filter
-// (nn = 1) comes here only for restrictions of many real functions, see
-// staged(); its other calls run in transformers_linear.hip.
+// (nn = 1) comes here only for some large calls, see staged(); its other calls
+// run in transformers_linear.hip.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -709,23 +709,20 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
     thr = ((thr + 63) / 64) * 64;
     int64_t nblocks = nbands * (int64_t)g.nyt * g.nxc;
     GH_REQUIRE(nblocks < (1ll << 31), GH_ERR_SHAPE, "transformer: too many blocks");
-    if constexpr (K == 2) {
-        // the short filter's interpolation and its other restrictions:
-        // transformers_linear.hip
-        constexpr int VEC = 16 / sizeof(V);
-        hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R, VEC>), dim3((unsigned)nblocks),
-                           dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
-    } else if (h->interp)
-        hipLaunchKernelGGL((interpolate_kernel<V, S, K, PPT_I>), dim3((unsigned)nblocks),
-                           dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
-    else if (constexpr int VEC = 16 / sizeof(V);
-             VEC > 1 && g.vec == VEC && ((uintptr_t)in & 15u) == 0)
-        hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R, (VEC > 1 ? VEC : 1)>),
-                           dim3((unsigned)nblocks), dim3(thr), lds, st, (const V*)in,
-                           (V*)out, g, ph, (S)alpha);
-    else
+    // the short filter's other calls do not come here, see staged()
+    constexpr int VEC = 16 / sizeof(V);
+    if (h->interp) {
+        if constexpr (K > 2 || sizeof(V) > 4)
+            hipLaunchKernelGGL((interpolate_kernel<V, S, K, PPT_I>), dim3((unsigned)nblocks),
+                               dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
+    } else if (VEC > 1 && g.vec == VEC && ((uintptr_t)in & 15u) == 0) {
+        if constexpr (VEC > 1)
+            hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R, VEC>), dim3((unsigned)nblocks),
+                               dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
+    } else if constexpr (K > 2) {
         hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R>), dim3((unsigned)nblocks),
                            dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
+    }
     GH_CHECK_LAUNCH();
     return GH_OK;
 }
@@ -734,9 +731,7 @@ template <typename V, typename S>
 int launch_k(const gh_transformer* h, const void* in, void* out, int64_t nb,
              const double* ph, double al, hipStream_t st) {
     switch (h->nn) {
-        case 1:
-            if constexpr (!is_complex<V>::value) return launch_t<V, S, 2>(h, in, out, nb, ph, al, st);
-            break;
+        case 1: return launch_t<V, S, 2>(h, in, out, nb, ph, al, st);
         case 2: return launch_t<V, S, 4>(h, in, out, nb, ph, al, st);
         case 3: return launch_t<V, S, 6>(h, in, out, nb, ph, al, st);
         case 4: return launch_t<V, S, 8>(h, in, out, nb, ph, al, st);
@@ -867,16 +862,33 @@ int64_t transformer_out_points(const gh_transformer* h) {
 
 namespace {
 
-// Restriction with the short filter of many real functions whose rows are
-// whole 16-byte vectors: beyond the 256 MB of the last-level cache the staged
-// kernel's single read of the input wins.  FP64, 16 x 112^3 (22 M points)
-// staged 36.3 us, not staged 35.3; 200 x 64^3 (52 M) 107 and 132; FP32, 64 x
-// 64^3 (17 M) 20.8 and 21.1, 256 x 64^3 68 and 105.  Complex data gain from
-// it nowhere (complex64, 200 x 64^3, k along x 147 and 139).
-bool staged(const gh_transformer* h, const void* in, int64_t nbands) {
-    return !h->interp && (h->dtype == GH_F64 || h->dtype == GH_F32) &&
-           h->g.vec == 16 / dtype_size(h->dtype) && ((uintptr_t)in & 15u) == 0 &&
-           nbands * transformer_in_points(h) > 24000000;
+// Short-filter calls that the staged kernels take, us staged / not staged.
+// Restrictions of more than 24 M points whose rows are whole 16-byte vectors
+// of 4- or 8-byte elements without y and z phases: beyond the 256 MB of the
+// last-level cache their single read of the input wins.  FP64, 16 x 112^3
+// (22 M) 36 / 35, 200 x 64^3 107 / 132, 256 x 112^3 682 / 751; FP32, 64 x 64^3
+// (17 M) 21 / 21, 256 x 112^3 364 / 571; complex64, k along x, 32 x 112^3 92 /
+// 108, 256 x 112^3 687 / 759, but with a phase along y 128 x 112^3 485 / 383;
+// complex128 128 x 112^3 667 / 686 and 757 / 689.
+// Interpolations to more than 18 M points of complex128 (one point per thread
+// there), or of FP64 rows of odd length (their 16-byte stores are not
+// aligned): complex128, to 40 x 72 x 68 x 68 (13 M) 50 / 46, to 16 x 112^3 (22
+// M) 86 / 126, to 256 x 112^3 1208 / 1691; FP64, to 95 x 95 x 111 x 8 (8 M) 27
+// / 17, to 128 x 111 x 111 x 115 445 / 507; others 603 / 451 (FP32, 256 x
+// 112^3) to 857 / 840 (FP64).
+bool staged(const gh_transformer* h, const void* in, int64_t nbands, const double* phase_cd) {
+    const int vs = dtype_size(h->dtype);
+    if (h->interp)
+        return (h->dtype == GH_C128 || (h->dtype == GH_F64 && h->g.m[2] % 2)) &&
+               nbands * transformer_out_points(h) > 18000000;
+    if (vs > 8 || h->g.vec != 16 / vs || ((uintptr_t)in & 15u) ||
+        nbands * transformer_in_points(h) <= 24000000)
+        return false;
+    const Phases ph = make_phases(phase_cd);
+    for (int c = 1; c < 3; c++)
+        for (int d = 0; d < 2; d++)
+            if (h->dtype == GH_C64 && (ph.re[c][d] != 1.0 || ph.im[c][d] != 0.0)) return false;
+    return true;
 }
 
 // Rows longer than a block of the staged kernels are refused for every filter.
@@ -912,7 +924,7 @@ int transformer_apply_scaled(const gh_transformer* h, const void* in_dev,
     GH_REQUIRE(in_dev && out_dev, GH_ERR_ARG, "transformer_apply: null argument");
     GH_REQUIRE(in_dev != out_dev, GH_ERR_ARG, "transformer_apply: in and out must differ");
     LinearMap lin;
-    if (transformer_linear(h, h->dtype, &lin) && !staged(h, in_dev, nbands)) {
+    if (transformer_linear(h, h->dtype, &lin) && !staged(h, in_dev, nbands, phase_cd)) {
         GH_REQUIRE(lin_rows_fit(h), GH_ERR_UNSUPPORTED,
                    "transformer: grid rows too long for one block");
         return linear_map(h->dtype, lin, in_dev, out_dev, nullptr, nbands, phase_cd, al, st);

@@ -12,8 +12,7 @@
 //   16 x 48^3 FP32 r   8.4 ->  7.3    16 x 24^3 FP32 i 8.5 ->  5.5
 //   40 x 72 x 66 x 68 complex128 r 60 -> 35, i back 50 -> 46
 //   64 x 56^3 i        227 -> 206     100 x 40 x 44 x 48 FP32 i 117 -> 94
-// Restriction of many real functions stays staged (staged() in
-// transformers.hip).
+// Some large calls stay staged (staged() in transformers.hip).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

@@ -54,3 +54,29 @@ def test_tiles(N_c, pbc, nn, dtype, tol, nb):
                 1j * ref.apply(x[i:i + 1].imag.astype(np.float64), None)
         got = out[i:i + 1].cpu().numpy()
         assert abs(got - want).max() <= tol * abs(want).max()
+
+
+# calls large enough for the staged kernels of the short filter: restriction
+# of whole vectors, complex128 and odd FP64 rows interpolated; the same bits
+# as a few bands alone, which take the other kernels (real data; complex128
+# with phases: last bits)
+@pytest.mark.parametrize('dtype,N_c,pbc,op,nb', [
+    (np.float64, (48, 44, 40), True, 'r', 290), (np.float32, (48, 44, 40), True, 'r', 290),
+    (np.complex64, (48, 44, 40), True, 'r', 290), (np.complex128, (48, 44, 36), True, 'i', 240),
+    (np.float64, (48, 44, 40), False, 'i', 230)])
+def test_large_calls(dtype, N_c, pbc, op, nb):
+    N_c = np.array(N_c)
+    gd = GridDescriptor(N_c, N_c * 0.3, (pbc,) * 3)
+    ogd = og.Grid(N_c, N_c * 0.3, pbc_c=(pbc,) * 3)
+    cplx = np.dtype(dtype).kind == 'c'
+    ph = ogd.phase_cd((0.25, 0, 0)) if cplx and pbc else None
+    a, b = (gd, gd.coarsen()) if op == 'r' else (gd.coarsen(), gd)
+    g = torch.Generator(device='cuda').manual_seed(3)
+    td = torch.from_numpy(np.zeros(1, dtype)).dtype
+    x = torch.randn((nb,) + tuple(int(k) for k in a.n_c), generator=g, dtype=td, device='cuda')
+    T = Transformer(a, b, 1, dtype)
+    out = T.apply(x, phases=ph)
+    for i in (0, nb // 2, nb - 1):
+        alone = T.apply(x[i:i + 1].contiguous(), phases=ph)
+        err = (out[i:i + 1] - alone).abs().max()
+        assert err <= (1e-15 if dtype == np.complex128 else 0) * alone.abs().max()
