@@ -589,8 +589,8 @@ template <typename V, typename S, bool HAS_V, bool HAS_SRC>
 __global__ void __launch_bounds__(256)
 stencil_generic_kernel(const V* __restrict__ in, V* __restrict__ out,
                        const S* __restrict__ vt, const V* __restrict__ src,
-                       S beta, S gamma, GenericArgs<S> a, PhaseArgs<S> ph,
-                       int64_t total) {
+                       S beta, S gamma, const double* __restrict__ eps, GenericArgs<S> a,
+                       PhaseArgs<S> ph, int64_t total) {
     const size_t npts = (size_t)a.n0 * a.n1 * a.n2;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
          t += (int64_t)gridDim.x * blockDim.x) {
@@ -606,7 +606,8 @@ stencil_generic_kernel(const V* __restrict__ in, V* __restrict__ out,
                          fetch_wrapped(inb, x + a.off[p][0], y + a.off[p][1],
                                        z + a.off[p][2], a, ph),
                          acc);
-        if (gamma != (S)0) acc = fma_rs(gamma, inb[gi], acc);
+        const S gb = eps ? gamma - (S)eps[band] : gamma;
+        if (gb != (S)0) acc = fma_rs(gb, inb[gi], acc);
         if (HAS_V) acc = fma_rs(vt[gi], inb[gi], acc);
         if (HAS_SRC) acc = fma_rs(beta, src[t], acc);
         out[t] = acc;
@@ -667,6 +668,7 @@ struct gh_stencil {
     int pbc[3];
     int R;          // max |offset| per axis (padding of the reference)
     bool cfd;
+    bool narrow;    // a periodic axis has fewer than R points
     double diag;
     // cfd representation
     double c0;
@@ -773,7 +775,7 @@ template <typename V, typename S>
 int launch_generic(const gh_stencil* h, const void* in, void* out,
                    int64_t nbands, const double* phase_cd, const void* vt,
                    const void* src, double beta, double alpha, double gamma,
-                   hipStream_t st) {
+                   const double* eps, hipStream_t st) {
     GenericArgs<S> a;
     a.np = (int)h->coefs.size();
     a.n0 = (int)h->n[0]; a.n1 = (int)h->n[1]; a.n2 = (int)h->n[2];
@@ -789,16 +791,16 @@ int launch_generic(const gh_stencil* h, const void* in, void* out,
     const V* srcp = (const V*)src;
     if (vt && src)
         hipLaunchKernelGGL((stencil_generic_kernel<V, S, true, true>), dim3(nblk), dim3(256), 0, st,
-                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, a, ph, total);
+                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, eps, a, ph, total);
     else if (vt)
         hipLaunchKernelGGL((stencil_generic_kernel<V, S, true, false>), dim3(nblk), dim3(256), 0, st,
-                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, a, ph, total);
+                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, eps, a, ph, total);
     else if (src)
         hipLaunchKernelGGL((stencil_generic_kernel<V, S, false, true>), dim3(nblk), dim3(256), 0, st,
-                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, a, ph, total);
+                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, eps, a, ph, total);
     else
         hipLaunchKernelGGL((stencil_generic_kernel<V, S, false, false>), dim3(nblk), dim3(256), 0, st,
-                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, a, ph, total);
+                           (const V*)in, (V*)out, vtp, srcp, (S)beta, (S)gamma, eps, a, ph, total);
     GH_CHECK_LAUNCH();
     return GH_OK;
 }
@@ -1024,6 +1026,14 @@ int gh_stencil_create(gh_stencil** out, int ncoefs, const double* coefs,
     } else {
         h->cfd = false;
     }
+    // The kernels for stencils along the axes read R neighbours on every axis
+    // and wrap an index once, while each offset was checked against its own
+    // axis only: a radius 3 along x is no longer than a domain with one
+    // periodic point along y, whose neighbours at 3 lie three periods away.
+    // The generic kernel reads the stencil's own points alone.
+    h->narrow = false;
+    for (int c = 0; c < 3; c++)
+        if (h->cfd && h->pbc[c] && h->n[c] < h->R) h->narrow = true;
     *out = h;
     return GH_OK;
 }
@@ -1165,6 +1175,9 @@ int gh_stencil_relax_from(const gh_stencil* h, void* f_dev, const void* s_dev, v
 
 struct gh_stencil_batch {
     BatchPlan plan;
+    // a batch with a narrow cell: its cells, which then run one by one
+    std::vector<gh_stencil> cells;
+    std::vector<int64_t> nbands;
 };
 
 int gh_stencil_batch_create(gh_stencil_batch** out, int ncells, const gh_stencil* const* ops,
@@ -1206,6 +1219,12 @@ int gh_stencil_batch_create(gh_stencil_batch** out, int ncells, const gh_stencil
         if (bp.counters) (void)hipFree(bp.counters);
         delete b;
         return rc;
+    }
+    bool narrow = false;
+    for (int c = 0; c < ncells; c++) narrow = narrow || ops[c]->narrow;
+    if (narrow) {
+        for (int c = 0; c < ncells; c++) b->cells.push_back(*ops[c]);
+        b->nbands.assign(nbands, nbands + ncells);
     }
     *out = b;
     return GH_OK;
@@ -1251,6 +1270,13 @@ int gh_stencil_batch_apply(const gh_stencil_batch* b, const void* const* in_dev,
     }
     hipStream_t st = (hipStream_t)stream;
     const void* const* vt = bp.has_v ? vt_dev : nullptr;
+    for (size_t c = 0; c < b->cells.size(); c++) {
+        const int rc = stencil_apply_full(&b->cells[c], in_dev[c], out_dev[c], b->nbands[c], nullptr,
+                                          vt ? vt[c] : nullptr, nullptr, 0.0, 1.0, 0.0, nullptr,
+                                          st);
+        if (rc != GH_OK) return rc;
+    }
+    if (!b->cells.empty()) return GH_OK;
 #define GH_RUN(V, S)                                                            \
     switch (bp.R) {                                                            \
         case 1: return launch_batch<V, S, 1>(bp, in_dev, out_dev, vt, st);      \
@@ -1270,7 +1296,7 @@ int64_t stencil_points(const gh_stencil* h) { return h->n[0] * h->n[1] * h->n[2]
 int stencil_dtype(const gh_stencil* h) { return h->dtype; }
 
 bool stencil_axes(const gh_stencil* h, DirectStencil* out) {
-    if (!h->cfd || h->mode != 0) return false;
+    if (!h->cfd || h->narrow || h->mode != 0) return false;
     *out = axes_of(h);
     return true;
 }
@@ -1292,7 +1318,9 @@ int stencil_apply_full(const gh_stencil* h, const void* in_dev, void* out_dev,
     if (nbands == 0) return GH_OK;  // empty arrays may carry null pointers
     GH_REQUIRE(in_dev && out_dev, GH_ERR_ARG, "stencil_apply: null argument");
     GH_REQUIRE(in_dev != out_dev, GH_ERR_ARG, "stencil_apply: in and out must differ");
-    if (h->cfd) {
+    GH_REQUIRE(!eps || h->cfd, GH_ERR_UNSUPPORTED,
+               "stencil_apply: per-band shift needs an orthogonal stencil");
+    if (h->cfd && !h->narrow) {
         switch (h->dtype) {
             case GH_F64: return launch_cfd<double, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
             case GH_C128: return launch_cfd<cplx<double>, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
@@ -1300,13 +1328,11 @@ int stencil_apply_full(const gh_stencil* h, const void* in_dev, void* out_dev,
             case GH_C64: return launch_cfd<cplx<float>, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
         }
     } else {
-        GH_REQUIRE(!eps, GH_ERR_UNSUPPORTED,
-                   "stencil_apply: per-band shift needs an orthogonal stencil");
         switch (h->dtype) {
-            case GH_F64: return launch_generic<double, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, st);
-            case GH_C128: return launch_generic<cplx<double>, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, st);
-            case GH_F32: return launch_generic<float, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, st);
-            case GH_C64: return launch_generic<cplx<float>, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, st);
+            case GH_F64: return launch_generic<double, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_C128: return launch_generic<cplx<double>, double>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_F32: return launch_generic<float, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
+            case GH_C64: return launch_generic<cplx<float>, float>(h, in_dev, out_dev, nbands, phase_cd, vt_dev, src_dev, beta, al, ga, eps, st);
         }
     }
     set_error("stencil_apply: bad dtype");
