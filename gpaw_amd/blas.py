@@ -108,7 +108,8 @@ def rotate(U, psi):
     64 x 64)."""
     m, k = U.shape
     if (psi.dtype != torch.float64 or U.dtype != torch.float64
-            or not psi.is_cuda or psi.dim() != 2 or not psi.is_contiguous()
+            or not psi.is_cuda or U.device != psi.device or U.is_neg()
+            or psi.is_neg() or psi.dim() != 2 or not psi.is_contiguous()
             or not 1 <= m <= 64 or not 1 <= k <= 64 or psi.shape[0] != k
             or psi.shape[1] >= 2**27
             or U.requires_grad or psi.requires_grad):

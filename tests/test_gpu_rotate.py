@@ -32,3 +32,23 @@ def test_transposed_and_infinite():
     want = U.T @ psi
     assert torch.equal(torch.isinf(out), torch.isinf(want))
     assert bool((torch.isinf(out).sum(0) == 30 * (torch.arange(50) == 7)).all())
+
+
+@pytest.mark.parametrize('n', [100, 10000])
+def test_other_devices_are_refused(n):
+    """A matrix or functions in host memory: an error, as for U @ psi."""
+    U = torch.ones(4, 4, dtype=torch.float64)
+    psi = torch.ones(4, n, dtype=torch.float64)
+    for a, b in ((U, psi.cuda()), (U.cuda(), psi)):
+        with pytest.raises(RuntimeError):
+            blas.rotate(a, b)
+
+
+@pytest.mark.parametrize('n', [100, 10000])
+def test_negated_views(n):
+    """Views that carry a pending sign (the imaginary part of a conjugate)."""
+    g = torch.Generator().manual_seed(3)
+    z = torch.randn(1, 1, generator=g, dtype=torch.complex128).cuda()
+    U = z.conj().imag
+    psi = torch.randn(1, n, generator=g, dtype=torch.float64).cuda()
+    assert torch.equal(blas.rotate(U, psi), -z.imag * psi)
