@@ -105,13 +105,16 @@ def rotate(U, psi):
     """U psi for the rows of psi: up to 64 FP64 functions on the framework's
     matrix-core kernel, else torch's product (for 64 functions of 64^3 points
     146 us against 70; that kernel keeps U in registers, which end at
-    64 x 64)."""
+    64 x 64).  Rows of fewer than 8192 points: torch's product, whose call
+    costs less (us per call, torch and the kernel: 16 functions of 1728
+    points 8.3 and 8.7, of 13824 10.8 and 8.9; 64 functions 8.1 and 12.3,
+    15.7 and 13.1; one wave needs 7 us for a tile of 64 x 64)."""
     m, k = U.shape
     if (psi.dtype != torch.float64 or U.dtype != torch.float64
             or not psi.is_cuda or U.device != psi.device or U.is_neg()
             or psi.is_neg() or psi.dim() != 2 or not psi.is_contiguous()
             or not 1 <= m <= 64 or not 1 <= k <= 64 or psi.shape[0] != k
-            or psi.shape[1] >= 2**27
+            or not 8192 <= psi.shape[1] < 2**27
             or U.requires_grad or psi.requires_grad):
         return U @ psi
     U = U.contiguous()

@@ -101,9 +101,12 @@ extern "C" int gh_rotate(int m, int k, int64_t n, const double* U_dev, const dou
     int ncu = 0;
     const int rc = device_cu_count(&ncu);
     if (rc != GH_OK) return rc;
-    // two blocks per CU (registers), each wave with many tiles
+    // two blocks per CU (registers), each wave with many tiles; a few
+    // functions leave so little in flight per wave that eight are needed
+    // (2 x 2, 1.4 M points: 37 us with two, 21 with eight)
     const int64_t tiles = (n + 15) / 16;
-    const unsigned blocks = (unsigned)std::min<int64_t>((tiles + 3) / 4, 2 * ncu);
+    const unsigned blocks =
+        (unsigned)std::min<int64_t>((tiles + 3) / 4, (m + k <= 16 ? 8 : 2) * ncu);
     const int ks = (k + 15) / 16, mt = (m + 15) / 16;
     hipStream_t st = (hipStream_t)stream;
 #define GH_ROT(MT, KB)                                                                  \

@@ -6,7 +6,8 @@ import pytest
 torch = pytest.importorskip('torch')
 pytestmark = pytest.mark.gpu
 
-from gpaw_amd import blas  # noqa: E402
+from gpaw_amd import _lib, blas  # noqa: E402
+from gpaw_amd._arrays import stream_ptr  # noqa: E402
 
 
 # k products of order one: k roundings of 1.1e-16 of at most k
@@ -32,6 +33,28 @@ def test_transposed_and_infinite():
     want = U.T @ psi
     assert torch.equal(torch.isinf(out), torch.isinf(want))
     assert bool((torch.isinf(out).sum(0) == 30 * (torch.arange(50) == 7)).all())
+
+
+def rotate_kernel(U, psi):
+    out = torch.full((U.shape[0], psi.shape[1]), float('nan'),
+                     dtype=torch.float64, device='cuda')
+    U, psi = U.contiguous().cuda(), psi.cuda()
+    _lib.check(_lib.lib().gh_rotate(*U.shape, psi.shape[1], U.data_ptr(),
+                                    psi.data_ptr(), out.data_ptr(),
+                                    stream_ptr()))
+    return out.cpu()
+
+
+@pytest.mark.parametrize('m,k', [(1, 1), (2, 2), (3, 5), (16, 16), (17, 15),
+                                 (48, 33), (64, 64), (10, 64), (64, 1)])
+@pytest.mark.parametrize('n', [1, 15, 17, 8191, 300007])
+def test_kernel(m, k, n):
+    """The kernel itself, also where rotate() takes the library's product."""
+    g = torch.Generator().manual_seed(m * 100 + k)
+    U = torch.randn(m, k, generator=g, dtype=torch.float64)
+    psi = torch.randn(k, n, generator=g, dtype=torch.float64)
+    out, want = rotate_kernel(U, psi), U @ psi
+    assert (out - want).abs().max() <= 1.1e-16 * k * (k + 12)
 
 
 @pytest.mark.parametrize('n', [100, 10000])
