@@ -71,6 +71,16 @@ __device__ __forceinline__ cplx<S> mul_phase(cplx<S> a, S pre, S pim) {
     return {a.re * pre - a.im * pim, a.re * pim + a.im * pre};
 }
 
+// The same where p is (1, 0) but for images: other lanes leave the other
+// component out, since an infinity times 0 is NaN.
+template <typename S>
+__device__ __forceinline__ S mul_phase_of(bool, S a, S, S) { return a; }
+template <typename S>
+__device__ __forceinline__ cplx<S> mul_phase_of(bool image, cplx<S> a, S pre, S pim) {
+    const S re = image ? a.re : (S)0, im = image ? a.im : (S)0;
+    return {a.re * pre - im * pim, re * pim + a.im * pre};
+}
+
 __device__ __forceinline__ double vadd(double a, double b) { return a + b; }
 __device__ __forceinline__ float vadd(float a, float b) { return a + b; }
 template <typename S>

@@ -156,7 +156,7 @@ stencil_direct_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __
                     const bool wr = (yout >> j) & 1;
                     const S pr = wr ? g.re[1][d] : (S)1, pi = wr ? g.im[1][d] : (S)0;
 #pragma unroll
-                    for (int i = 0; i < PT; i++) yv[j].v[i] = mul_phase(yv[j].v[i], pr, pi);
+                    for (int i = 0; i < PT; i++) yv[j].v[i] = mul_phase_of(wr, yv[j].v[i], pr, pi);
                 }
             }
         }

@@ -281,11 +281,12 @@ stencil_rows_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __re
         if constexpr (CPLX) {
             const S pr = low ? g.re[c][1] : high ? g.re[c][0] : (S)1;
             const S pi = low ? g.im[c][1] : high ? g.im[c][0] : (S)0;
+            const bool image = low || high;      // see mul_phase_of
 #pragma unroll
             for (int i = 0; i < PT; i++) {
                 const S a = v[2 * i], b = v[2 * i + 1];
-                v[2 * i] = a * pr - b * pi;
-                v[2 * i + 1] = a * pi + b * pr;
+                v[2 * i] = a * pr - (image ? b : (S)0) * pi;
+                v[2 * i + 1] = (image ? a : (S)0) * pi + b * pr;
             }
         }
         return v;
@@ -316,8 +317,8 @@ stencil_rows_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __re
     auto z_ghost = [&](V v, int zz) {
         if (!CPLX || !g.zphase) return v;
         const bool low = zz < 0, high = zz >= n2;
-        return mul_phase(v, low ? g.re[2][1] : high ? g.re[2][0] : (S)1,
-                         low ? g.im[2][1] : high ? g.im[2][0] : (S)0);
+        return mul_phase_of(low || high, v, low ? g.re[2][1] : high ? g.re[2][0] : (S)1,
+                            low ? g.im[2][1] : high ? g.im[2][0] : (S)0);
     };
     barrier_only();
 #pragma unroll

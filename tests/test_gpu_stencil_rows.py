@@ -156,3 +156,39 @@ def test_unsymmetric_coefficients(monkeypatch, N_c, pbc, nb, dtype, k_c,
     op.apply(d, out, ph)
     tol = 2e-5 if dtype in (np.float32, np.complex64) else 1e-12
     assert abs(out[pick].cpu().numpy() - ref).max() < tol * abs(ref).max()
+
+
+@pytest.mark.parametrize('kernel', ['', 'rows', 'reg'])
+@pytest.mark.parametrize('dtype', [np.complex128, np.complex64])
+@pytest.mark.parametrize('N_c', [(9, 10, 12), (9, 10, 11), (40, 44, 46)])
+@pytest.mark.parametrize('axis', [0, 1, 2])
+def test_bloch_phases_keep_infinities_apart(monkeypatch, N_c, dtype, kernel,
+                                            axis):
+    """An infinite real part at a face gives the imaginary part nothing but
+    through a Bloch phase: only the points that read it as a periodic image
+    have both parts infinite."""
+    monkeypatch.setenv('GPAW_AMD_STENCIL', kernel)
+    N_c = np.array(N_c)
+    gd = GridDescriptor(N_c, N_c * 0.4, True)
+    at = [n // 2 for n in N_c]
+    at[axis] = 0
+    nb = 1 if N_c[0] < 40 else 10
+    a = np.ones((nb,) + tuple(gd.n_c), dtype)
+    a[(0,) + tuple(at)] = np.inf + 0j
+    op = Laplace(gd, -0.5, 3, dtype)
+    d = torch.from_numpy(a).cuda()
+    out = torch.empty_like(d)
+    op.apply(d, out, gd.phase_cd((0.2, 0.15, -0.1)))
+    out = out.cpu().numpy()
+    re, im = np.zeros(a.shape, bool), np.zeros(a.shape, bool)
+    for c in range(3):
+        for j in range(-3, 4):
+            p = list(at)
+            p[c] += j
+            image = p[c] < 0
+            p[c] %= N_c[c]
+            re[(0,) + tuple(p)] = True
+            if image:
+                im[(0,) + tuple(p)] = True
+    assert (~np.isfinite(out.real) == re).all()
+    assert (~np.isfinite(out.imag) == im).all()
