@@ -27,6 +27,7 @@
 //   64 x 72 x 80 x 90 complex128, general k   465 -> 281  (208)
 //   256 x 112^3 float32            712 ->  632  (564)
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -508,27 +509,50 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
     // about 6 KB at a CU's share of the HBM rate) plus the bytes of a plane
     // (ghost rows come from L2 and count half) of every block that its CU
     // runs beside it; blocks beyond what the CUs hold go into further rounds.
+    // One row count for each number of tiles and one run length for each number
+    // of runs: the choice of all pairs, at 4 to 20 % of the host time (1 us
+    // per call at 16 x 48^3, 6 at 2 x 256 x 256 x 24).
+    struct Run { int lx, nxc; };
+    Run runs[192];
+    int nruns = 0;
+    if (h.planes > 0) {
+        const int lx = std::min(h.planes, g.n0);
+        runs[nruns++] = Run{lx, (g.n0 + lx - 1) / lx};
+    } else {
+        for (int nxc = 1; nxc <= std::max(1, g.n0 / (2 * R)) && nruns < 192;) {
+            const int lx = (g.n0 + nxc - 1) / nxc;
+            runs[nruns++] = Run{lx, (g.n0 + lx - 1) / lx};
+            if (lx == 1) break;
+            nxc = std::max(nxc + nxc / 16, (g.n0 + lx - 2) / (lx - 1));
+        }
+    }
+    auto fits = [&](int ty) {
+        return lds_of(ty) <= kLdsBytes - 1024 && (comp_of(ty) + kDepth * g.lw) * 64 <= kMaxThreads;
+    };
     double best = 0;
+    int nyt_last = 0;
     g.ty = 0;
-    for (int ty = 1; ty <= g.n1; ty++) {
-        if (lds_of(ty) > kLdsBytes - 1024 || (comp_of(ty) + kDepth * g.lw) * 64 > kMaxThreads) break;
+    for (int ty = 1; ty <= g.n1 && fits(ty); ty++) {
         if (h.rows > 0 && ty != std::min(h.rows, g.n1)) continue;
-        const int64_t nyt = (g.n1 + ty - 1) / ty;
+        const int nyt = (g.n1 + ty - 1) / ty;
+        if (nyt == nyt_last) continue;
+        nyt_last = nyt;
         const int threads = (comp_of(ty) + kDepth * g.lw) * 64;
-        const int64_t fit = std::max(1, std::min(1024 / threads, (int)(kLdsBytes / lds_of(ty))));
-        for (int nxc = 1; nxc <= std::max(1, g.n0 / (2 * R)); nxc++) {
-            const int lx = h.planes > 0 ? std::min(h.planes, g.n0) : (g.n0 + nxc - 1) / nxc;
-            const int64_t blocks = nbands * nyt * ((g.n0 + lx - 1) / lx);
-            const int64_t rounds = (blocks + ncu * fit - 1) / (ncu * fit);
-            const int64_t beside = std::min<int64_t>(fit, (blocks + ncu - 1) / ncu);
-            const double t = (double)rounds * (lx + R + 2) *
-                             (beside * (2.0 * ty + R) * g.n2 * sizeof(V) + 6144.0);
+        const double fit = std::max(1, std::min(1024 / threads, (int)(kLdsBytes / lds_of(ty))));
+        const double tiles = (double)nbands * nyt, bytes = (2.0 * ty + R) * g.n2 * sizeof(V);
+        // (the small number keeps whole quotients whole)
+        const double per_room = 1.0 / (ncu * fit), per_cu = 1.0 / ncu;
+        for (int k = 0; k < nruns; k++) {
+            const double blocks = tiles * runs[k].nxc;
+            const double rounds = std::ceil(blocks * per_room - 1e-9);
+            const double beside = std::min(fit, std::ceil(blocks * per_cu - 1e-9));
+            const double t = rounds * (runs[k].lx + R + 2) * (beside * bytes + 6144.0);
             if (g.ty == 0 || t < best) {
                 best = t;
                 g.ty = ty;
-                g.lx = lx;
+                g.lx = runs[k].lx;
             }
-            if (h.planes > 0 || blocks > 8 * ncu * fit) break;
+            if (rounds > 8) break;
         }
     }
     if (g.ty == 0) return GH_ERR_UNSUPPORTED;
