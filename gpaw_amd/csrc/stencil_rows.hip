@@ -533,7 +533,8 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
     int nyt_last = 0;
     g.ty = 0;
     for (int ty = 1; ty <= g.n1 && fits(ty); ty++) {
-        if (h.rows > 0 && ty != std::min(h.rows, g.n1)) continue;
+        // rows that were asked for: as many of them as fit
+        if (h.rows > 0 && ty < std::min(h.rows, g.n1) && ty < g.n1 && fits(ty + 1)) continue;
         const int nyt = (g.n1 + ty - 1) / ty;
         if (nyt == nyt_last) continue;
         nyt_last = nyt;
@@ -554,6 +555,7 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
             }
             if (rounds > 8) break;
         }
+        if (h.rows > 0) break;
     }
     if (g.ty == 0) return GH_ERR_UNSUPPORTED;
     g.nyt = (g.n1 + g.ty - 1) / g.ty;
