@@ -33,7 +33,7 @@ int stencil_direct(int dtype, const DirectStencil& h, const void* in, void* out,
                    const void* src, double beta, double alpha, double gamma,
                    const double* eps, hipStream_t st);
 
-// The LDS ring (stencil_rows.hip): stencils of radius 1..3, rows of any length and alignment, any Bloch phases;
+// The LDS ring (stencil_rows.hip): stencils of radius 1..6, rows of any length and alignment, any Bloch phases;
 // GH_ERR_UNSUPPORTED where no tile fits
 int stencil_rows(int dtype, const DirectStencil& h, const void* in, void* out,
                  int64_t nbands, const double* phase_cd, const void* vt,

@@ -761,7 +761,11 @@ int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
     // FP64, R = 3, 2 x 64^3 (4.2 MB) 7.3 against 8.6 us, 96^3 (7.1 MB) 9.8
     // against 8.6, 64 x 24^3 (7.1 MB) 10.9 against 8.1.
     const int64_t bytes = nb * h->n[0] * h->n[1] * h->n[2] * (int64_t)sizeof(V);
-    if (h->mode == 2 || (h->mode == 0 && bytes > 5 * 1024 * 1024)) {
+    // FP32 rows that are not whole vectors, radius 4 or 5: the ring's reads at
+    // element alignment cost more than its LDS saves (64 x 95 x 95 x 103 278
+    // against 311 us at R = 4, 322 against 356 at 5; 490 against 404 at 6).
+    const bool loses = h->dtype == GH_F32 && h->n[2] % 4 && (h->R == 4 || h->R == 5);
+    if (h->mode == 2 || (h->mode == 0 && bytes > 5 * 1024 * 1024 && !loses)) {
         int ncu = 0;
         int rc = device_cu_count(&ncu);
         if (rc != GH_OK) return rc;

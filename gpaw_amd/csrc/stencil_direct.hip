@@ -1,7 +1,6 @@
 // Finite-difference stencils along the grid axes without LDS: the form for
-// grids the LDS-ring kernel cannot take or cannot fill the GPU with (rows
-// that are not 16-byte multiples, such as the odd rows of cells with zero
-// boundaries, radii above 3, one or a few small grids).
+// grids that the LDS ring (stencil_rows.hip) cannot fill the GPU with, one or
+// a few small ones, and for rows too long for its tiles.
 //
 // A thread owns PT z-adjacent points (16 bytes) of one row and marches along
 // x with a register queue of the 2R + 1 planes; the y and z neighbours come

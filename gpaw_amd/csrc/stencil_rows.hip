@@ -1,6 +1,6 @@
 // Finite-difference stencils along the grid axes: an LDS ring of x-planes, for
 // rows of any length and alignment, every element type, boundary and Bloch
-// phase (radius 1 to 3).
+// phase (radius 1 to 6).
 //
 // A block owns one band, a tile of ty full (y, z) rows and a run of
 // x-planes.  Loader wavefronts stream the tile's rows and its 2R ghost rows
@@ -37,7 +37,11 @@ namespace gh {
 
 namespace {
 
-constexpr int kMaxThreads = 1024;
+// Radii above 3 need up to 235 registers: half the threads, without scratch.
+// T + v, R = 4 and 6, us, the kernel without LDS and here: 64 x 96^3 float64 554
+// -> 391, 758 -> 334; 32 x 96^3 complex128, general k 1011 -> 386, 1436 -> 1434;
+// 64 x 64^3 complex128, k along x 587 -> 252, 737 -> 370.
+template <int R> constexpr int kMaxThreads = R > 3 ? 512 : 1024;
 constexpr size_t kLdsBytes = 160 * 1024;
 constexpr int kDepth = 2;         // planes in flight
 
@@ -108,7 +112,7 @@ __device__ __forceinline__ void load_n(const V* p, V* v) {
 // Laplacian), so half of them are live.
 template <typename V, typename S, int R, int PT, bool ALIGNED, bool SYM, bool HAS_V,
           bool HAS_SRC>
-__global__ void __launch_bounds__(kMaxThreads)
+__global__ void __launch_bounds__(kMaxThreads<R>)
 stencil_rows_kernel(const V* __restrict__ in, V* __restrict__ out, const S* __restrict__ vt,
                     const V* src, S beta, RowsArgs<S, R> g) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -527,7 +531,7 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
         }
     }
     auto fits = [&](int ty) {
-        return lds_of(ty) <= kLdsBytes - 1024 && (comp_of(ty) + kDepth * g.lw) * 64 <= kMaxThreads;
+        return lds_of(ty) <= kLdsBytes - 1024 && (comp_of(ty) + kDepth * g.lw) * 64 <= kMaxThreads<R>;
     };
     double best = 0;
     int nyt_last = 0;
@@ -603,6 +607,9 @@ int launch(const DirectStencil& h, const void* in, void* out, int64_t nb, const 
         case 1: return launch_r<V, S, 1>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
         case 2: return launch_r<V, S, 2>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
         case 3: return launch_r<V, S, 3>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
+        case 4: return launch_r<V, S, 4>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
+        case 5: return launch_r<V, S, 5>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
+        case 6: return launch_r<V, S, 6>(h, in, out, nb, ph, vt, src, beta, al, ga, eps, ncu, st);
     }
     return GH_ERR_UNSUPPORTED;
 }
