@@ -32,6 +32,7 @@
 // the instruction), the same permutation for A and B, so each lane reads W
 // contiguous elements with 16-byte LDS reads.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -360,23 +361,23 @@ gram_small_kernel(const char* __restrict__ A, const char* __restrict__ B, int64_
 
 // C[i][j] = alpha * sum over chunks (FP64, a fixed order) of the partial
 // blocks; Hermitian mode forms i >= j and writes its mirror image too;
-// conj_out conjugates.  A block sums 16 neighbouring outputs, 16 chunks at a
-// time: at 64 bands a thread per output left 16 blocks to walk about 1000
-// chunks one after the other (339 us; with the 64-row form's 256 chunks now
-// under 17 us).
-constexpr int kRedOut = 16;
-
-template <typename T, bool CPLX, int BM, int BN>
+// conj_out conjugates.  A block sums NO neighbouring outputs, 256 / NO chunks
+// at a time, 16 outputs where there are many chunks: at 64 bands a thread per
+// output left 16 blocks to walk about 1000 chunks one after the other (339
+// us; with the 64-row form's 256 chunks now under 17 us).  Many bands have few
+// chunks, and 16 outputs would leave threads without one (1000 x 1000 float32
+// over 1728 points, 3 chunks, product and sum: 73 us with 16, 52 with 256).
+template <typename T, bool CPLX, int BM, int BN, int NO>
 __global__ void __launch_bounds__(256)
 gram_reduce_kernel(const T* __restrict__ work, int m, int n, int herm, int nJ,
                    int nchunks, double alpha, int conj_out, int i0,
                    double* __restrict__ C) {
     constexpr int NC = CPLX ? 2 : 1;
-    constexpr int NG = 256 / kRedOut;
-    __shared__ double red[NC][NG][kRedOut + 1];
-    const int jl = threadIdx.x % kRedOut, grp = threadIdx.x / kRedOut;
-    const int i = i0 + (int)blockIdx.y, j = blockIdx.x * kRedOut + jl;
-    if (herm && i < (int)blockIdx.x * kRedOut) return;   // the whole block is above
+    constexpr int NG = 256 / NO;
+    __shared__ double red[NC][NG][NO + 1];
+    const int jl = threadIdx.x % NO, grp = threadIdx.x / NO;
+    const int i = i0 + (int)blockIdx.y, j = blockIdx.x * NO + jl;
+    if (herm && i < (int)blockIdx.x * NO) return;   // the whole block is above
     const bool live = j < n && (!herm || j <= i);
     double re = 0.0, im = 0.0;
     if (live) {
@@ -457,10 +458,16 @@ int launch_gram_reduce(const GramPlan& pl, int m, int n, double alpha, int herm,
     const int nchunks = pl.nseg > 0 ? pl.nchunks : 0;
     for (int i0 = 0; i0 < m; i0 += (int)kBandSlice) {   // one grid row per output row
         const int mi = std::min<int>((int)kBandSlice, m - i0);
-        hipLaunchKernelGGL((gram_reduce_kernel<T, CPLX, BM, BN>),
-                           dim3((unsigned)((n + kRedOut - 1) / kRedOut), (unsigned)mi),
-                           dim3(256), 0, st, (const T*)work, m, n, herm, pl.nJ, nchunks, alpha,
-                           conj_out, i0, C);
+        auto go = [&](auto outputs) {
+            constexpr int NO = decltype(outputs)::value;
+            hipLaunchKernelGGL((gram_reduce_kernel<T, CPLX, BM, BN, NO>),
+                               dim3((unsigned)((n + NO - 1) / NO), (unsigned)mi), dim3(256), 0,
+                               st, (const T*)work, m, n, herm, pl.nJ, nchunks, alpha, conj_out, i0,
+                               C);
+        };
+        if (nchunks > 16 || n <= 16) go(std::integral_constant<int, 16>{});
+        else if (nchunks > 4 || n <= 64) go(std::integral_constant<int, 64>{});
+        else go(std::integral_constant<int, 256>{});
         GH_CHECK_LAUNCH();
     }
     return GH_OK;

@@ -25,7 +25,7 @@ namespace gh {
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kMaxThreads = 256;
 
 template <typename S>
 struct LinArgs {
@@ -39,7 +39,7 @@ struct LinArgs {
 template <typename V> struct Nine { V v[3][3]; };
 
 template <typename V, typename S>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kMaxThreads)
 restrict_linear_kernel(const V* __restrict__ in, V* __restrict__ out, LinArgs<S> a) {
     constexpr bool CPLX = is_complex<V>::value;
     const LinGrid<S>& g = a.g;
@@ -48,7 +48,7 @@ restrict_linear_kernel(const V* __restrict__ in, V* __restrict__ out, LinArgs<S>
     const int xc = rem / a.nblk;
     const int npts = a.m[1] * a.m[2];
     // threads beyond the plane repeat its last point
-    const int p = min((rem - xc * a.nblk) * kThreads + (int)threadIdx.x, npts - 1);
+    const int p = min((rem - xc * a.nblk) * (int)blockDim.x + (int)threadIdx.x, npts - 1);
     const int y = p / a.m[2], z = p - y * a.m[2];
     const size_t plane = (size_t)g.n[1] * g.n[2];
     const V* __restrict__ inb = in + (size_t)band * g.n[0] * plane;
@@ -133,7 +133,7 @@ restrict_linear_kernel(const V* __restrict__ in, V* __restrict__ out, LinArgs<S>
 
 // out = alpha I(in) or, with BASE, base + alpha I(in) (base may be out)
 template <typename V, typename S, bool BASE>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kMaxThreads)
 interpolate_linear_kernel(const V* __restrict__ in, V* out, const V* base, LinArgs<S> a) {
     constexpr int PT = 16 / (int)sizeof(V);
     typedef LinPoints<V, S, PT> Points;
@@ -146,7 +146,7 @@ interpolate_linear_kernel(const V* __restrict__ in, V* out, const V* base, LinAr
     const int per = a.nblk * a.nxc, band = L / per, rem = L - band * per;
     const int xc = rem / a.nblk;
     const int nv = (a.m[2] + PT - 1) / PT;
-    const int p = (rem - xc * a.nblk) * kThreads + (int)threadIdx.x;
+    const int p = (rem - xc * a.nblk) * (int)blockDim.x + (int)threadIdx.x;
     if (p >= a.m[1] * nv) return;
     const int y = p / nv, z = (p - y * nv) * PT;
     const bool part = z + PT > a.m[2];               // the row ends inside the vector
@@ -209,12 +209,23 @@ int launch(const LinearMap& h, const void* in, void* out, const void* base, int6
     if (crc != GH_OK) return crc;
     const int64_t threads = (int64_t)h.m[1] * (h.interp ? (h.m[2] + PT - 1) / PT : h.m[2]);
     const int steps = h.interp ? ((h.m[0] - 1 + h.skip[0]) >> 1) - (h.skip[0] >> 1) + 1 : h.m[0];
-    a.nblk = (int)((threads + kThreads - 1) / kThreads);
+    // Threads of a block: what leaves the fewest idle ones on a plane (8 x 8
+    // points kept three waves of four idle).
+    int tb = kMaxThreads;
+    double least = 0;
+    for (int t = kMaxThreads; t >= 64; t -= 64) {
+        const double padded = (double)((threads + t - 1) / t * t) * (1.0 + 1e-4 * (kMaxThreads - t));
+        if (t == kMaxThreads || padded < least) {
+            least = padded;
+            tb = t;
+        }
+    }
+    a.nblk = (int)((threads + tb - 1) / tb);
     // The run along x with the least estimated time: a step costs about as
     // much as the first plane of a run (latency), rounds of the blocks that
     // the GPU holds (6 per CU by registers).
     double best = 0;
-    const double room = 6.0 * ncu;
+    const double room = 6.0 * ncu * kMaxThreads / tb;
     for (int nxc = 1; nxc <= steps; nxc += 1 + nxc / 8) {
         const int lx = (steps + nxc - 1) / nxc;
         const double blocks = (double)nbands * a.nblk * ((steps + lx - 1) / lx);
@@ -229,7 +240,7 @@ int launch(const LinearMap& h, const void* in, void* out, const void* base, int6
     a.nxc = (steps + a.lx - 1) / a.lx;
     const int64_t nblocks = nbands * (int64_t)a.nblk * a.nxc;
     GH_REQUIRE(nblocks < (1ll << 31), GH_ERR_SHAPE, "transformer: too many blocks");
-    const dim3 grid((unsigned)nblocks), block(kThreads);
+    const dim3 grid((unsigned)nblocks), block(tb);
     if (!h.interp)
         hipLaunchKernelGGL((restrict_linear_kernel<V, S>), grid, block, 0, st, (const V*)in,
                            (V*)out, a);

@@ -123,3 +123,24 @@ def test_gram_views_and_errors():
     assert float(((c - ref).abs() / bound(w, w)).max()) < 1e-13
     with pytest.raises(ValueError):
         blas.gram(a[:10], a[:12], hermitian=True)
+
+
+@pytest.mark.parametrize('dtype', DTYPES)
+@pytest.mark.parametrize('m,n,k', [(300, 517, 40), (517, 300, 1728),
+                                   (200, 65, 6000), (520, 520, 640),
+                                   (257, 257, 13824)])
+@pytest.mark.parametrize('conj', [False, True])
+def test_gram_few_chunks(dtype, m, n, k, conj):
+    """Few chunks per result: the sum with 256, 64 and 16 results per block,
+    at the ends of its blocks, general and Hermitian."""
+    g = torch.Generator(device='cuda')
+    g.manual_seed(m + k)
+    a = torch.randn((m, k), dtype=dtype, device='cuda', generator=g)
+    b = torch.randn((n, k), dtype=dtype, device='cuda', generator=g)
+    c = blas.gram(a, b, alpha=0.7, conj=conj)
+    err = (c - exact(a, b, 0.7, conj)).abs() / bound(a, b)
+    assert float(err.max()) < tol(dtype)
+    c = blas.gram(a, alpha=0.7, hermitian=True, conj=conj)
+    err = (c - exact(a, a, 0.7, conj)).abs() / bound(a, a)
+    assert float(err.max()) < tol(dtype)
+    assert torch.equal(c, c.conj().T)
