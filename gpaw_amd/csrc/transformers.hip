@@ -617,16 +617,19 @@ constexpr int ppt_of(bool interp) {
 
 // Tile (output rows) and x-run of a block: the pair with the least estimated
 // time.  A block walks its run's input planes (the first ones only prime the
-// filter queue).  A plane costs what every block beside it on the CU moves
-// through HBM and, at a fifteenth, through LDS, or, if that is longer, the
-// latency of its two barriers and its loads: 0.8 us (restriction) or 1.6
-// (interpolation) and 0.17 per load of a thread, four times that where every
-// element's phase is worked out; in bytes at a CU's share of the HBM rate
-// (20 KB per us).  Blocks beyond what the CUs hold go into further rounds.
-// Cutting the runs until 2048 blocks existed, as before, primed 9 to 11
-// planes for every 8: 2 densities 112^3 -> 224^3 with nn = 3 took 119 us and
-// take 61, 128 complex64 functions restricted from 112^3 684 and 520 us, 3 of
-// 46 x 40 x 44 with a general k 69 and 44.
+// filter queue).  A plane costs what the blocks that share its CU move, HBM
+// bytes and 0.35 of the LDS bytes of the filters at 30 KB per us, and, on top
+// of that, the latency of its two barriers, of its loads (more where every
+// element's phase is worked out) and of its filters' passes over the block.  A
+// CU holds 1024 threads (registers).  Of restricted rows two thirds of the
+// halo's bytes come from the caches.  The constants are those that choose best
+// among the measured tiles of 580 calls (every type, nn = 1..4, 0.5 MB to 2
+// GB): 4 % above the fastest tile on average, 9 % with the constants before
+// and 60 % with whole-divisor tiles and runs cut until there were 2048
+// blocks.  us, those, the constants before and here: nn = 4, float32, 50 x 15
+// x 17 x 19 interpolated 17, 27, 16; nn = 3, float64, 16 x 56^3 interpolated 110,
+// 51, 51; nn = 2, float64, 16 x 112^3 restricted 58, 71, 57, complex64, 128 x 63^3
+// 108, 153, 109.
 struct TTile {
     int tj = 0, lx = 0, nry = 0;
     size_t lds = 0;
@@ -638,6 +641,15 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
     const int K = 2 * h->nn;
     TTile best;
     double tbest = 0;
+    // Short restrictions come here only when they are large (staged()): blocks of
+    // up to 12 rows and 256 threads and runs of about five planes, whose
+    // neighbours then read the same rows at nearly the same time, are 7 %
+    // above the fastest tile on average (26 % at most, 64 calls); the estimate
+    // is 11 % above it (53 %), whole-divisor tiles with long runs 44 %.
+    const bool brief = !h->interp && h->nn == 1;
+    const int brief_runs = std::max(1, (g.m[0] + 2) / 5);
+    const int brief_lx = (g.m[0] + brief_runs - 1) / brief_runs;
+    int last = 0;
     for (int tj = 1; tj <= g.m[1]; tj++) {
         const int nry = h->interp ? (tj + 1) / 2 + 2 * h->nn + 1 : 2 * tj + 2 * K - 3;
         // interpolation: staged rows + their z-filtered rows; restriction:
@@ -646,25 +658,44 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
                                      : (size_t)(nry + tj) * g.zw * vsize;
         const int thr = ((tj * g.m[2] + ppt - 1) / ppt + 63) / 64 * 64;
         if (lds > 64 * 1024 || thr > 1024) break;
-        const int64_t nyt = (g.m[1] + tj - 1) / tj;
-        const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(2048 / thr, 160 * 1024 / lds));
-        const double hbm = ((double)nry * g.zw +
-                            (h->interp ? 2.0 : 0.5) * tj * g.m[2]) * vsize;
-        const double taps = h->interp ? (K + 2) / 2.0 * (nry * g.m[2] + tj * g.m[2])
-                                      : (K + 2.0) * (tj * g.zw + tj * g.m[2]);
-        const double plane = hbm + taps * vsize / 15;
-        const double loads = std::ceil((double)nry * g.zw / (h->interp ? 1 : g.vec) / thr);
-        const double fixed = (h->interp ? 32e3 : 16e3) + 3.4e3 * loads * (phases ? 4 : 1);
-        const double room = (double)ncu * fit;
+        const int nyt = (g.m[1] + tj - 1) / tj;
+        if (nyt == last) continue;      // the same tiles, fuller
+        last = nyt;
+        if (brief) {
+            if (tj > 1 && (thr > 256 || tj > 12)) break;
+            best.tj = tj;
+            best.lx = brief_lx;
+            best.nry = nry;
+            best.lds = lds;
+            continue;
+        }
+        const double fit = std::max(1, std::min(1024 / thr, (int)(160 * 1024 / lds)));
+        // filtered elements: along z of the staged rows (interpolation) or
+        // along y (restriction), then the output points
+        const double out = (double)tj * g.m[2], staged = (double)nry * g.zw;
+        const double first = h->interp ? (double)nry * g.m[2] : (double)tj * g.zw;
+        const double own = (double)std::min(2 * tj, nry) * g.zw;
+        const double read = h->interp ? staged : own + 0.35 * (staged - own);
+        const double bytes = (read + (h->interp ? 2.0 : 0.5) * out +
+                              0.35 * (h->interp ? 0.5 : 1.0) * (K + 2) * (first + out)) * vsize;
+        const double loads = std::ceil(staged / (h->interp ? 1 : g.vec) / thr);
+        const double passes = std::ceil(first / thr);
+        const double latency =
+            h->interp ? 0.65 + 0.15 * loads * (phases ? 4 : 1) + 0.45 * passes
+                      : 0.7 + 0.6 * loads * (phases ? 6 : 1) + 0.35 * passes;
+        const double per_room = 1.0 / (ncu * fit), per_cu = 1.0 / ncu;
         // steps of an eighth: a few microseconds per call for this search
         for (int nxc = 1; nxc <= std::max(1, g.m[0] / 2); nxc += 1 + nxc / 8) {
-            const int lx = (g.m[0] + nxc - 1) / nxc;
-            const double blocks = (double)(nbands * nyt) * ((g.m[0] + lx - 1) / lx);
-            const double rounds = std::ceil(blocks / room);
-            const double beside = std::min((double)fit, std::ceil(blocks / ncu));
+            int lx = (g.m[0] + nxc - 1) / nxc;
+            if (h->interp && nxc > 1) lx += lx & 1;     // fine planes come in pairs
+            const int runs = (g.m[0] + lx - 1) / lx;
+            const double blocks = (double)nbands * nyt * runs;
+            const double rounds = std::ceil(blocks * per_room - 1e-9);
+            const double beside = std::min(fit, std::ceil(blocks * per_cu - 1e-9));
             const double planes = h->interp ? (lx + 1) / 2 + K - 1 : 2 * lx + 2 * K - 3;
-            const double bytes = beside * plane;
-            const double t = rounds * planes * (std::max(bytes, fixed) + 0.2 * std::min(bytes, fixed));
+            // (blocks of later rounds start as those of earlier ones end)
+            const double t = (0.35 * std::max(1.0, blocks * per_room) + 0.65 * rounds) * planes *
+                             (beside * bytes / 30e3 + latency);
             if (best.tj == 0 || t < tbest) {
                 tbest = t;
                 best.tj = tj;
@@ -672,7 +703,7 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
                 best.nry = nry;
                 best.lds = lds;
             }
-            if (rounds > 4) break;
+            if (rounds > 8) break;
         }
     }
     return best;
@@ -712,9 +743,8 @@ int launch_t(const gh_transformer* h, const void* in, void* out,
     // the short filter's other calls do not come here, see staged()
     constexpr int VEC = 16 / sizeof(V);
     if (h->interp) {
-        if constexpr (K > 2 || sizeof(V) > 4)
-            hipLaunchKernelGGL((interpolate_kernel<V, S, K, PPT_I>), dim3((unsigned)nblocks),
-                               dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
+        hipLaunchKernelGGL((interpolate_kernel<V, S, K, PPT_I>), dim3((unsigned)nblocks),
+                           dim3(thr), lds, st, (const V*)in, (V*)out, g, ph, (S)alpha);
     } else if (VEC > 1 && g.vec == VEC && ((uintptr_t)in & 15u) == 0) {
         if constexpr (VEC > 1)
             hipLaunchKernelGGL((restrict_kernel<V, S, K, PPT_R, VEC>), dim3((unsigned)nblocks),
@@ -862,27 +892,34 @@ int64_t transformer_out_points(const gh_transformer* h) {
 
 namespace {
 
-// Short-filter calls that the staged kernels take, us staged / not staged.
-// Restrictions of more than 24 M points whose rows are whole 16-byte vectors
-// of 4- or 8-byte elements without y and z phases: beyond the 256 MB of the
-// last-level cache their single read of the input wins.  FP64, 16 x 112^3
-// (22 M) 36 / 35, 200 x 64^3 107 / 132, 256 x 112^3 682 / 751; FP32, 64 x 64^3
-// (17 M) 21 / 21, 256 x 112^3 364 / 571; complex64, k along x, 32 x 112^3 92 /
-// 108, 256 x 112^3 687 / 759, but with a phase along y 128 x 112^3 485 / 383;
-// complex128 128 x 112^3 667 / 686 and 757 / 689.
-// Interpolations to more than 18 M points of complex128 (one point per thread
-// there), or of FP64 rows of odd length (their 16-byte stores are not
-// aligned): complex128, to 40 x 72 x 68 x 68 (13 M) 50 / 46, to 16 x 112^3 (22
-// M) 86 / 126, to 256 x 112^3 1208 / 1691; FP64, to 95 x 95 x 111 x 8 (8 M) 27
-// / 17, to 128 x 111 x 111 x 115 445 / 507; others 603 / 451 (FP32, 256 x
-// 112^3) to 857 / 840 (FP64).
+// Short-filter calls that the staged kernels take, us staged / not staged, each
+// with its best tile (larger calls repeat the last ratio).
+// Restrictions whose rows are whole 16-byte vectors of 4- or 8-byte elements
+// without y and z phases: once the input is beyond the caches, their single
+// read of it wins.  FP32 above 60 MB (the other kernel's 4-byte loads cost as
+// many instructions as 16-byte ones): 30 x 64^3 (31 MB) 22 / 13, 19 x 94 x 94 x
+// 92 (61) 22 / 23, 26 x 120^3 (179) 47 / 60, 659 x 60^3 (569) 140 / 241.  FP64
+// above 260 MB: 16 x 98^3 (120) 31 / 25, 41 x 92^3 (255) 62 / 63, 499 x 46^3 (388)
+// 95 / 110.  complex64 above 380 MB: 36 x 96^3 (254) 76 / 62, 231 x 58^3 (360)
+// 104 / 103, 664 x 58^3 (1036) 263 / 281, with a phase along y 721 x 32 x 126 x
+// 16 (355) 193 / 104.  complex128 never (one element per load either way; 138
+// x 78 x 78 x 112, 1435 MB, 343 / 365, but 84 x 34 x 142 x 48 24 / 18).
+// Interpolations to more than 240 MB of complex128 (one point per thread not
+// staged): 124 x 53 x 11 x 26 (229) 57 / 59, 22 x 53 x 38 x 67 (362) 98 / 118,
+// 377 x 27^3 (906) 218 / 273; 92 x 17 x 11 x 59 (134) 33 / 30.  To more than 800
+// MB of real rows that are not whole vectors (their stores are not aligned):
+// FP64 2001 x 8 x 14 x 53 (805) 288 / 322, FP32 769 x 51 x 61 x 11 (855) 359 /
+// 426, 4961 x 19^3 (1123) 420 / 592; FP32 71 x 53^3 (332) 150 / 141.
 bool staged(const gh_transformer* h, const void* in, int64_t nbands, const double* phase_cd) {
     const int vs = dtype_size(h->dtype);
-    if (h->interp)
-        return (h->dtype == GH_C128 || (h->dtype == GH_F64 && h->g.m[2] % 2)) &&
-               nbands * transformer_out_points(h) > 18000000;
+    if (h->interp) {
+        const int64_t bytes = nbands * transformer_out_points(h) * vs;
+        if (h->dtype == GH_C128) return bytes > 240000000;
+        return h->dtype != GH_C64 && h->g.m[2] * vs % 16 && bytes > 800000000;
+    }
     if (vs > 8 || h->g.vec != 16 / vs || ((uintptr_t)in & 15u) ||
-        nbands * transformer_in_points(h) <= 24000000)
+        nbands * transformer_in_points(h) * vs <=
+            (vs == 4 ? 60000000 : h->dtype == GH_F64 ? 260000000 : 380000000))
         return false;
     const Phases ph = make_phases(phase_cd);
     for (int c = 1; c < 3; c++)
