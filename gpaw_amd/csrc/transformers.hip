@@ -641,12 +641,14 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
     const int K = 2 * h->nn;
     TTile best;
     double tbest = 0;
-    // Short restrictions come here only when they are large (staged()): blocks of
-    // up to 12 rows and 256 threads and runs of about five planes, whose
+    // Short restrictions come here only when they are large (staged()).  Beyond
+    // the 256 MB of the last-level cache blocks of up to 12 rows and 256 threads and runs of about five planes, whose
     // neighbours then read the same rows at nearly the same time, are 7 %
     // above the fastest tile on average (26 % at most, 64 calls); the estimate
-    // is 11 % above it (53 %), whole-divisor tiles with long runs 44 %.
-    const bool brief = !h->interp && h->nn == 1;
+    // is 11 % above it (53 %), whole-divisor tiles with long runs 44 %.  Within
+    // it the estimate is better: float32, 95 x 64^3 25 us against 31.
+    const bool brief = !h->interp && h->nn == 1 &&
+                       nbands * g.n[0] * g.n[1] * g.n[2] * vsize > 260000000;
     const int brief_runs = std::max(1, (g.m[0] + 2) / 5);
     const int brief_lx = (g.m[0] + brief_runs - 1) / brief_runs;
     int last = 0;
