@@ -41,7 +41,6 @@ constexpr int kMaxGeneric = 96; // stencil points of the generic kernel
 template <typename S>
 struct CfdCoefs {
     S c0;
-    const double* eps;  // per band: centre coefficient c0 - eps[band] (or null)
     S cm[3][kMaxR];  // coefficient of offset -(j+1) along axis c
     S cp[3][kMaxR];  // coefficient of offset +(j+1) along axis c
 };
@@ -81,9 +80,8 @@ __device__ __forceinline__ V load_x(const V* __restrict__ inb, int x, int yz,
 // with vmcnt(0) just before the barrier of the iteration that first reads
 // it.  Compute wavefronts never write LDS: they refill the x register queue
 // from the ring, read y/z neighbours from the current plane's slot, apply
-// Bloch phases / zero ghosts at read time, and store H psi.  The potential
-// (and src) at their own points come from plain loads issued before the
-// LDS work of the plane: the potential is shared by every band and stays in
+// zero ghosts at read time, and store H psi.  The potential at their own points
+// comes from plain loads issued before the LDS work of the plane: the potential is shared by every band and stays in
 // L2, and a DMA ring for it measured 15% slower than these loads.
 constexpr int kRingMaxThreads = 1024;
 constexpr int kDmaBytes = 16;              // bytes per lane per DMA op
@@ -135,11 +133,9 @@ __device__ __forceinline__ void ring_block_coords(const RingGeom& rg, int L,
 // block's waves split into rg.ncomp compute and rg.nload loader wavefronts;
 // waves beyond those (a batched launch sized for a larger tile) only take
 // part in the barriers.
-template <typename V, typename S, int R, int PPT, bool HAS_V, bool HAS_SRC,
-          bool SYM>
+template <typename V, typename S, int R, int PPT, bool HAS_V, bool SYM>
 __device__ __forceinline__ void
-ring_tile(const V* __restrict__ in, V* __restrict__ out,
-          const S* __restrict__ vt, const V* __restrict__ src, S beta,
+ring_tile(const V* __restrict__ in, V* __restrict__ out, const S* __restrict__ vt,
           const CfdCoefs<S>& cf, const RingGeom& rg, const PhaseArgs<S>& ph,
           int L, V* __restrict__ ring) {
     const CfdGeom& g = rg.g;
@@ -148,7 +144,6 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
     const int n2 = g.n2;
     int band, xc, yt;
     ring_block_coords(rg, L, band, xc, yt);
-    const S c0b = cf.eps ? cf.c0 - (S)cf.eps[band] : cf.c0;
     const int y0 = yt * g.ty;
     const int tye = min(g.ty, g.n1 - y0);
     const int x0 = xc * g.lx;
@@ -260,7 +255,7 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
             q[j] = V4{load_x(inb, x0 - R + j, yz, g, ph), load_x(inb, x0 - R + j, yz + 1, g, ph),
                       load_x(inb, x0 - R + j, yz + 2, g, ph),
                       load_x(inb, x0 - R + j, yz + 3, g, ph)};
-        S k0 = c0b;
+        S k0 = cf.c0;
         S km[3][R], kp[3][R];
         if (SYM) asm volatile("" : "+v"(k0));
 #pragma unroll
@@ -283,9 +278,8 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                     q[2 * R] = v;
                 }
                 const size_t gi = (size_t)x * plane + yz;
-                V4 vv, ss;
+                V4 vv;
                 if (HAS_V) vv = *reinterpret_cast<const V4*>(vt + gi);
-                if (HAS_SRC) ss = *reinterpret_cast<const V4*>(src + band * bstride + gi);
                 const V4* sl = reinterpret_cast<const V4*>(ring + ((x - x0) % P) * slot);
                 V4 acc = q[R] * k0;
 #pragma unroll
@@ -336,7 +330,6 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                     }
                 acc = V4{a4[0], a4[1], a4[2], a4[3]};
                 if (HAS_V) acc = vv * q[R] + acc;
-                if (HAS_SRC) acc = ss * beta + acc;
                 if (act) {
                     V4* o = reinterpret_cast<V4*>(outb + gi);
                     __builtin_nontemporal_store(acc, o);
@@ -398,7 +391,7 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
         // is full in this loop and would spill them through v_readlane)
         // (symmetric stencils only: with both signs pinned the register
         // file overflows)
-        S k0 = c0b;
+        S k0 = cf.c0;
         S km[3][R], kp[3][R];
         if (SYM) asm volatile("" : "+v"(k0));
 #pragma unroll
@@ -421,9 +414,8 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                     q[2 * R] = v;
                 }
                 const size_t gi = (size_t)x * plane + yz;
-                V2 vv, ss;
+                V2 vv;
                 if (HAS_V) vv = *reinterpret_cast<const V2*>(vt + gi);
-                if (HAS_SRC) ss = *reinterpret_cast<const V2*>(src + band * bstride + gi);
                 const V2* sl = reinterpret_cast<const V2*>(ring + ((x - x0) % P) * slot);
                 V2 acc = q[R] * k0;
 #pragma unroll
@@ -478,7 +470,6 @@ ring_tile(const V* __restrict__ in, V* __restrict__ out,
                     }
                 }
                 if (HAS_V) acc = vv * q[R] + acc;
-                if (HAS_SRC) acc = ss * beta + acc;
                 if (act) {
                     V2* o = reinterpret_cast<V2*>(outb + gi);
                     __builtin_nontemporal_store(acc, o);
@@ -537,9 +528,8 @@ stencil_ring_batched_kernel(const RingCell<S>* __restrict__ cells, BatchPtrs<V, 
         for (int k = 1; k < ncells; k++)
             if (L >= cells[k].lbeg) c = k;
         const RingCell<S>& cell = cells[c];
-        ring_tile<V, S, R, PPT, HAS_V, false, SYM>(ptr.in[c], ptr.out[c], ptr.vt[c], nullptr,
-                                                    (S)0, cell.cf, cell.rg, cell.ph,
-                                                    L - cell.lbeg, ring);
+        ring_tile<V, S, R, PPT, HAS_V, SYM>(ptr.in[c], ptr.out[c], ptr.vt[c], cell.cf, cell.rg,
+                                            cell.ph, L - cell.lbeg, ring);
     }
     if (threadIdx.x == 0) {
         __threadfence();
@@ -677,7 +667,7 @@ struct gh_stencil {
     // generic representation
     std::vector<double> coefs;
     std::vector<int64_t> offs;
-    int ty_req = 0, lx_req = 0, depth_req = 0;
+    int ty_req = 0, lx_req = 0;
     int mode = 0;            // GPAW_AMD_STENCIL: 1 reg (the kernel without LDS), 2 rows
 };
 
@@ -872,7 +862,6 @@ int plan_batch(BatchPlan& bp, const gh_stencil* const* ops, const int64_t* nband
         rc.rg.nbands = (int)nbands[c];
         rc.rg.nlogical = (int)(nbands[c] * g.nyt);
         rc.cf.c0 = (S)h->c0;
-        rc.cf.eps = nullptr;
         for (int a = 0; a < 3; a++)
             for (int j = 0; j < kMaxR; j++) {
                 rc.cf.cm[a][j] = (S)h->cm[a][j];
@@ -1055,7 +1044,6 @@ int gh_stencil_set_tile(gh_stencil* h, int rows, int planes, int depth) {
                GH_ERR_ARG, "set_tile: bad args");
     h->ty_req = rows;
     h->lx_req = planes;
-    h->depth_req = depth;
     return GH_OK;
 }
 

@@ -174,8 +174,8 @@ class FDOperator:
         return self._lib.gh_stencil_diagonal(self.handle)
 
     def set_tile(self, rows=0, planes=0, depth=0):
-        """Tile shape of the stencil kernel: rows per block, x-planes per
-        block, prefetch depth of batched cells (0 = automatic)."""
+        """Tile shape of the stencil kernel: rows per block (as many as
+        fit), x-planes per block (0 = automatic); depth has no effect."""
         _lib.check(self._lib.gh_stencil_set_tile(self.handle, int(rows),
                                                  int(planes), int(depth)))
 

@@ -101,9 +101,9 @@ int gh_stencil_apply_shifted(const gh_stencil* h, const void* in_dev,
                              const double* eps_dev, void* stream);
 
 /* Tile choice of the stencil kernel: rows of the (y, z) tile per block,
- * planes per block along x; 0 = automatic.  depth: prefetch depth in planes
- * (2 or 3) of batched cells, without effect on a single grid.  Used by the
- * autotuner. */
+ * planes per block along x; 0 = automatic, more rows than a block holds are
+ * cut down.  depth (0, 2 or 3) has no effect: a single grid's prefetch depth is
+ * fixed, a batch is given its own.  Used by the autotuner. */
 int gh_stencil_set_tile(gh_stencil* h, int rows, int planes, int depth);
 
 /* Jacobi relaxation of L f = s in place (replaces Operator.relax,
