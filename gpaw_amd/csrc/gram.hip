@@ -249,12 +249,14 @@ gram_mfma_kernel(const char* __restrict__ A, const char* __restrict__ B,
 // Band counts up to 64 (both operands): the 128 x 128 block above would
 // spend three of its four waves on rows that do not exist, so here every
 // wave owns the whole 64 x 64 product of a k-slice (complex128: two waves
-// share a slice, 32 columns each, to fit the registers).  What bounds it is
-// the matrix-core rate (a 128-byte segment of 64 + 64 rows is 64
-// instructions for 16 KB), so one wave per SIMD with the next segment's
-// loads in flight suffices; the waves share no data and each lane's 16-byte
-// loads of a row use whole 128-byte lines, so there is no LDS stage and no
-// barrier in the loop.  In Hermitian mode tiles above the diagonal are
+// share a slice, 32 columns each, to fit the registers).  A 128-byte segment
+// of 64 + 64 rows is 64 instructions for 16 KB, more time on the matrix cores
+// than its loads take, so the registers go to one wave per SIMD with the next
+// segment's loads in flight.  At the size below it reaches 37 % of the matrix
+// rate, and its bytes would take 26 us (one operand) to 53 (two) at a copy's
+// rate: neither limits it; with one wave per SIMD, latency likely does.  The
+// waves share no data and each lane's 16-byte loads of a row use whole 128-byte
+// lines, so there is no LDS stage and no barrier in the loop.  In Hermitian mode tiles above the diagonal are
 // skipped.  The block's slices are added in FP64 through LDS and one partial
 // block per workgroup (always FP64) goes to the workspace.  64 FP64 bands of
 // 64^3 points: 182 us with the 128-row blocks, 73 us here (29 TFLOP/s of the

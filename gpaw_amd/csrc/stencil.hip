@@ -73,16 +73,16 @@ __device__ __forceinline__ V load_x(const V* __restrict__ inb, int x, int yz,
 
 // ------------------------------------------------- LDS-ring stencil --
 // The batched cells' form of the ring.  The block owns one band and a tile
-// of ty full (y, z) rows and marches along x; plane tiles (ty + 2R rows, ghosts included) are streamed HBM -> LDS by
-// global_load_lds DMA into a ring of P = R + D + 1 slots, D planes ahead of
+// of ty full (y, z) rows and marches along x; plane tiles (ty + 2R rows, ghosts
+// included) are streamed HBM -> LDS by global_load_lds DMA into a ring of P = R + D + 1 slots, D planes ahead of
 // use, by D loader wavefronts: loader w owns the planes xp with
 // (xp - x0) % D == w, so it has exactly one plane in flight and waits for it
 // with vmcnt(0) just before the barrier of the iteration that first reads
 // it.  Compute wavefronts never write LDS: they refill the x register queue
 // from the ring, read y/z neighbours from the current plane's slot, apply
 // zero ghosts at read time, and store H psi.  The potential at their own points
-// comes from plain loads issued before the LDS work of the plane: the potential is shared by every band and stays in
-// L2, and a DMA ring for it measured 15% slower than these loads.
+// comes from plain loads issued before the LDS work of the plane: it is shared
+// by every band and stays in L2, and a DMA ring for it measured 15% slower.
 constexpr int kRingMaxThreads = 1024;
 constexpr int kDmaBytes = 16;              // bytes per lane per DMA op
 

@@ -20,11 +20,12 @@
 // HBM bound for many bands (psi read, result written; ghost rows from L2).
 // T + v, R = 3, us, against the ring with one point per thread for complex
 // phases, its register-queue fallback for odd rows and fixed 16-row tiles:
-//   256 x 112^3 float64           1355 -> 1262  (copy of the bytes: 1128)
+//   256 x 112^3 float64           1355 -> 1262  (copy of the bytes: 1128; 1390 -> 1297
+//                                 between the other kernels of an H psi)
 //   64 x 96^3 float64              295 ->  195  (178)
 //   48 x 95 x 95 x 103, zero bc    418 ->  194  (140)
-//   128 x 96^3 complex64, k along x  580 -> 382, general k 1046 -> 402 (355)
-//   64 x 72 x 80 x 90 complex128, general k   465 -> 281  (208)
+//   128 x 96^3 complex64, k along x  580 -> 382, general k 1046 -> 411 (355)
+//   64 x 72 x 80 x 90 complex128, general k   465 -> 272  (208)
 //   256 x 112^3 float32            712 ->  632  (564)
 #include <algorithm>
 #include <cmath>
