@@ -751,11 +751,17 @@ int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
     // FP64, R = 3, 2 x 64^3 (4.2 MB) 7.3 against 8.6 us, 96^3 (7.1 MB) 9.8
     // against 8.6, 64 x 24^3 (7.1 MB) 10.9 against 8.1.
     const int64_t bytes = nb * h->n[0] * h->n[1] * h->n[2] * (int64_t)sizeof(V);
-    // FP32 rows that are not whole vectors, radius 4 or 5: the ring's reads at
-    // element alignment cost more than its LDS saves (64 x 95 x 95 x 103 278
-    // against 311 us at R = 4, 322 against 356 at 5; 490 against 404 at 6).
-    const bool loses = h->dtype == GH_F32 && h->n[2] % 4 && (h->R == 4 || h->R == 5);
-    if (h->mode == 2 || (h->mode == 0 && bytes > 5 * 1024 * 1024 && !loses)) {
+    // Radii above 3, whose ghost rows are most of a small tile: the ring for rows
+    // of whole 16-byte vectors and for complex64 planes of 16 rows and more.
+    // Other rows pay for reads at element alignment as well.  300 calls, ring
+    // over no LDS, median: whole vectors 0.52 (complex64, R = 4) to 0.88
+    // (complex128, 6); complex64 0.64 to 0.80, but 1.5 and 1.7 on 15 and 13 rows;
+    // FP64 0.94 to 1.02, up to 3.3 (64 x 27 x 13); FP32 1.1 to 1.4, up to 3.5.
+    // complex128 from 8 MB (2 x 57^3, 6 MB, R = 4: 15.0 against 12.3 us).
+    const bool suits = h->R <= 3 || h->n[2] * (int64_t)sizeof(V) % 16 == 0 ||
+                       (h->dtype == GH_C64 && h->n[1] >= 16);
+    const int64_t least = (h->R > 3 && h->dtype == GH_C128 ? 8 : 5) * 1024 * 1024;
+    if (h->mode == 2 || (h->mode == 0 && bytes > least && suits)) {
         int ncu = 0;
         int rc = device_cu_count(&ncu);
         if (rc != GH_OK) return rc;

@@ -562,7 +562,9 @@ int launch_r(const DirectStencil& h, const void* in, void* out, int64_t nbands,
         }
         if (h.rows > 0) break;
     }
-    if (g.ty == 0) return GH_ERR_UNSUPPORTED;
+    // (long complex128 rows leave a tile so few rows beside its 2R ghost rows
+    // that the kernel without LDS is faster: 115^3, R = 5, one row 73 us, 44)
+    if (g.ty == 0 || (R > 3 && h.rows == 0 && g.ty < std::min(R / 2, g.n1))) return GH_ERR_UNSUPPORTED;
     g.nyt = (g.n1 + g.ty - 1) / g.ty;
     g.nxc = (g.n0 + g.lx - 1) / g.lx;
     g.ncomp = comp_of(g.ty);
