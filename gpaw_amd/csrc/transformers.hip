@@ -621,15 +621,18 @@ constexpr int ppt_of(bool interp) {
 // bytes and 0.35 of the LDS bytes of the filters at 30 KB per us, and, on top
 // of that, the latency of its two barriers, of its loads (more where every
 // element's phase is worked out) and of its filters' passes over the block.  A
-// CU holds 1024 threads (registers).  Of restricted rows two thirds of the
-// halo's bytes come from the caches.  The constants are those that choose best
-// among the measured tiles of 580 calls (every type, nn = 1..4, 0.5 MB to 2
-// GB): 4 % above the fastest tile on average, 9 % with the constants before
-// and 60 % with whole-divisor tiles and runs cut until there were 2048
-// blocks.  us, those, the constants before and here: nn = 4, float32, 50 x 15
-// x 17 x 19 interpolated 17, 27, 16; nn = 3, float64, 16 x 56^3 interpolated 110,
-// 51, 51; nn = 2, float64, 16 x 112^3 restricted 58, 71, 57, complex64, 128 x 63^3
-// 108, 153, 109.
+// CU holds four waves on each of its four SIMDs (registers); blocks of more than
+// four waves take whole rounds of the SIMDs, so that two of five waves fit and
+// not three (us, where three were assumed and here: complex128, nn = 3, 53 x 72 x
+// 78 x 94 restricted 287, 175, 6 x 108 x 94 x 88 with a general k 147, 94).  Of
+// restricted rows two thirds of the halo's bytes come from the caches.  The
+// constants are those that choose best among the measured tiles of 1500 calls
+// (every type, nn = 1..4, 0.5 MB to 2 GB): 3 % above the fastest tile on
+// average, 9 % with the constants before and 60 % with whole-divisor tiles and
+// runs cut until there were 2048 blocks.  us, those, the constants before and
+// here: nn = 4, float32, 50 x 15 x 17 x 19 interpolated 17, 27, 16; nn = 3, float64,
+// 16 x 56^3 interpolated 110, 51, 51; nn = 2, float64, 16 x 112^3 restricted 58, 71,
+// 57, complex64, 128 x 63^3 108, 153, 109.
 struct TTile {
     int tj = 0, lx = 0, nry = 0;
     size_t lds = 0;
@@ -642,8 +645,9 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
     TTile best;
     double tbest = 0;
     // Short restrictions come here only when they are large (staged()).  Beyond
-    // the 256 MB of the last-level cache blocks of up to 12 rows and 256 threads and runs of about five planes, whose
-    // neighbours then read the same rows at nearly the same time, are 7 %
+    // the 256 MB of the last-level cache blocks of up to 12 rows and 256 threads
+    // and runs of about five planes, whose neighbours then read the same rows at
+    // nearly the same time, are 7 %
     // above the fastest tile on average (26 % at most, 64 calls); the estimate
     // is 11 % above it (53 %), whole-divisor tiles with long runs 44 %.  Within
     // it the estimate is better: float32, 95 x 64^3 25 us against 31.
@@ -671,7 +675,8 @@ TTile choose_tile(const gh_transformer* h, int vsize, int ppt, int64_t nbands, b
             best.lds = lds;
             continue;
         }
-        const double fit = std::max(1, std::min(1024 / thr, (int)(160 * 1024 / lds)));
+        const int waves = thr / 64, slots = waves <= 4 ? 16 / waves : 4 / ((waves + 3) / 4);
+        const double fit = std::max(1, std::min(slots, (int)(160 * 1024 / lds)));
         // filtered elements: along z of the staged rows (interpolation) or
         // along y (restriction), then the output points
         const double out = (double)tj * g.m[2], staged = (double)nry * g.zw;
