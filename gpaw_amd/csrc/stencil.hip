@@ -761,7 +761,17 @@ int launch_cfd(const gh_stencil* h, const void* in, void* out, int64_t nb,
     const bool suits = h->R <= 3 || h->n[2] * (int64_t)sizeof(V) % 16 == 0 ||
                        (h->dtype == GH_C64 && h->n[1] >= 16);
     const int64_t least = (h->R > 3 && h->dtype == GH_C128 ? 8 : 5) * 1024 * 1024;
-    if (h->mode == 2 || (h->mode == 0 && bytes > least && suits)) {
+    // A block of the ring holds rows of one plane, so planes of less than a wave
+    // of vectors, or two where rows end inside one, leave most of it idle, however
+    // many grids there are.  Ring over no LDS at 180 MB, R = 1, by vectors of a
+    // plane: whole rows (float64 and float32) 16 2.2, 32 1.3, 50 1.3, 56 0.8, 64
+    // 0.7, 98 0.5; others 28 4.5, 60 1.5, 66 1.5, 91 1.3, 120 1.0, 138 0.7, 190 0.6.
+    const int64_t vectors = h->n[1] * ((h->n[2] * (int64_t)sizeof(V) + 15) / 16);
+    // Periodic complex64, whose images cost the kernel without LDS more, from 32:
+    // 8 x 8 points 1.06, R = 2 0.78.
+    const int64_t whole = h->dtype == GH_C64 && (h->pbc[1] || h->pbc[2]) ? 32 : 56;
+    const bool fills = vectors >= (h->n[2] * (int64_t)sizeof(V) % 16 == 0 ? whole : 128);
+    if (h->mode == 2 || (h->mode == 0 && bytes > least && suits && fills)) {
         int ncu = 0;
         int rc = device_cu_count(&ncu);
         if (rc != GH_OK) return rc;
